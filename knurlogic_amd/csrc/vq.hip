@@ -19,6 +19,7 @@
 //
 // x is converted to fp16 for the dot products: exact for activations of
 // normal fp16 range (|x| < 65504; tiny values lose precision below 6e-5).
+#include "vq_gemm.hpp"
 #include "common.hpp"
 #include "qgemv.hpp"
 #include "vq_mfma.hpp"
@@ -424,14 +425,16 @@ int kmi_vq_glu(const void* x, int64_t T, int64_t H, int64_t I, int k, const int3
     return OK;
 }
 
-// Workspace: act [T*k, I], y [T*k, H] for the combine, then the expert sort
-// of the MFMA path (sized for up to 4096 experts).
+// Workspace: act [T*k, I], y [T*k, H] for the combine, the expert sort of the
+// MFMA paths (sized for up to 4096 experts), then x as fp16 [T, H] (the
+// grouped GEMM's).
 static size_t vq_act_bytes(int64_t T, int64_t I, int k) { return ((size_t)T * k * I * 2 + 255) & ~(size_t)255; }
 static size_t vq_y_bytes(int64_t T, int64_t H, int k) { return ((size_t)T * k * H * 2 + 255) & ~(size_t)255; }
 
 size_t kmi_vq_switch_glu_workspace_bytes(int64_t T, int64_t H, int64_t I, int k) {
     if (T <= 0 || H <= 0 || I <= 0 || k <= 0) return 0;
-    return vq_act_bytes(T, I, k) + vq_y_bytes(T, H, k) + sort_index_bytes(T * k, 4096, 1);   // any tile size
+    return vq_act_bytes(T, I, k) + vq_y_bytes(T, H, k) + sort_index_bytes(T * k, 4096, 1) +   // any tile size
+           (size_t)T * H * 2;
 }
 
 }  // extern "C"
@@ -494,8 +497,44 @@ static int vq_switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, in
     // inds from the router (every expert in range) and few pairs: the MFMA
     // kernels form their tiles themselves, no sort
     const bool formed = routed && !pair_mode && pair_tiles_fit(P, E, tile_rows);
+    // Prefill: rows grouped by expert in large tiles on the codebook GEMM
+    // (not where the router's call would form its tiles, so both calls agree)
+    const bool gemm = sortable && !pair_tiles_fit(P, E, tile_rows) && !pair_mode &&
+                      vqg_wanted(code_bytes, 8, P, avg) && al16(x) && al16(codes_gate) &&
+                      al16(codes_up) && al16(codes_down) && T * H * 2 < (1LL << 31) &&
+                      P * (H > I ? H : I) * 2 < (1LL << 31) &&
+                      vqg_supported(code_bytes, 0, 8, 0, E, I, H, kc, two_cb) &&
+                      vqg_supported(code_bytes, 0, 8, 0, E, H, I, kc, false);
     SortedRows sr = {};
     void* index_ws = (char*)workspace + vq_act_bytes(T, I, k) + vq_y_bytes(T, H, k);
+    if (gemm) {
+        const int tm = vqg_tile_rows(code_bytes, 8);
+        rc = launch_sort_rows(inds, P, 1, (int)E, tm, index_ws, y, H, st, &sr);
+        if (rc) return rc;
+        uint16_t* x16 = (uint16_t*)((char*)index_ws + sort_index_bytes(P, 4096, 1));
+        rc = launch_vqg_to_f16(x, T * H, x16, st);
+        if (rc) return rc;
+        VqgArgs g = {};
+        g.x = x16; g.xrows = T; g.lhs_div = k; g.tiles = sr.tiles; g.sorted = sr.sorted; g.E = E;
+        g.codes[0] = codes_gate; g.codes[1] = codes_up;
+        g.sc[0] = (const uint16_t*)scales_gate; g.sc[1] = (const uint16_t*)scales_up;
+        g.cb[0] = (const uint16_t*)codebook_gate; g.cb[1] = (const uint16_t*)codebook_up;
+        g.kc = kc; g.N = I; g.K = H; g.y = act; g.rows = P; g.y_f16 = 1;
+        rc = launch_vqg(g, code_bytes, 0, 8, true, sr.max_tiles, st);
+        if (rc) return rc;
+        KMI_CHECK_LAUNCH("vq_gemm(glu)");
+        VqgArgs d = g;
+        d.x = act; d.xrows = P; d.lhs_div = 1;
+        d.codes[0] = d.codes[1] = codes_down;
+        d.sc[0] = d.sc[1] = (const uint16_t*)scales_down;
+        d.cb[0] = d.cb[1] = (const uint16_t*)codebook_down;
+        d.N = H; d.K = I; d.y = y; d.y_f16 = 0;
+        rc = launch_vqg(d, code_bytes, 0, 8, false, sr.max_tiles, st);
+        if (rc) return rc;
+        KMI_CHECK_LAUNCH("vq_gemm(down)");
+        if (scores) return kmi_moe_combine(y, scores, dtype, T, k, H, out, stream);
+        return OK;
+    }
     if ((m_glu || m_down) && !pair_mode && !formed) {
         // the sort zeroes y's rows of out-of-range experts (no tile holds them)
         rc = launch_sort_rows(inds, P, 1, (int)E, tile_rows, index_ws, m_down ? y : nullptr, H, st, &sr);

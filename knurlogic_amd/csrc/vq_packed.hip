@@ -21,6 +21,7 @@
 // sums meet by cross-lane shuffles.  Scale groups are summed in fp32 and
 // scaled once per group.  With two row sets (gate and up) the epilogue is
 // Qwen3.5's _SwiGLU with its roundings.
+#include "vq_gemm.hpp"
 #include "common.hpp"
 #include "qgemv.hpp"
 #include "vq_packed_mfma.hpp"
@@ -648,15 +649,15 @@ int kmi_vq_packed_glu(const void* x, int64_t X, int64_t H, int64_t I, const uint
 }
 
 // SwitchGLU over packed VQ experts in one call.  Workspace: act [T*k, I],
-// y [T*k, H] for the combine, then the expert sort (sized for up to 4096
-// experts at any tile height).
+// y [T*k, H] for the combine, the expert sort (sized for up to 4096 experts
+// at any tile height), then x as fp16 [T, H] (the grouped GEMM's).
 static size_t vps_act_bytes(int64_t P, int64_t I) { return ((size_t)P * I * 2 + 255) & ~(size_t)255; }
 static size_t vps_y_bytes(int64_t P, int64_t H) { return ((size_t)P * H * 2 + 255) & ~(size_t)255; }
 
 size_t kmi_vq_packed_switch_glu_workspace_bytes(int64_t T, int64_t H, int64_t I, int k) {
     if (T <= 0 || H <= 0 || I <= 0 || k <= 0) return 0;
     const int64_t P = T * k;
-    return vps_act_bytes(P, I) + vps_y_bytes(P, H) + sort_index_bytes(P, 4096, 1);
+    return vps_act_bytes(P, I) + vps_y_bytes(P, H) + sort_index_bytes(P, 4096, 1) + (size_t)T * H * 2;
 }
 
 }  // extern "C"
@@ -729,6 +730,39 @@ static int vps_switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, i
         const bool formed = routed && pair_tiles_fit(P, E, tile_rows);
         SortedRows sr = {};
         int32_t* const list = (int32_t*)((char*)workspace + vps_act_bytes(P, I) + vps_y_bytes(P, H));
+        // Prefill: large expert tiles on the codebook GEMM (not where the
+        // router's call would form its tiles, so both calls agree)
+        if (!pair_tiles_fit(P, E, tile_rows) && vqg_wanted(0, dim, P, avg) && ((uintptr_t)x & 15u) == 0 &&
+            (((uintptr_t)scales_gate | (uintptr_t)scales_up | (uintptr_t)scales_down) & 3u) == 0 &&
+            I * Wg * 4 < (1LL << 31) && H * Wd * 4 < (1LL << 31) &&
+            vqg_supported(0, pack_bits, dim, group, E, I, H, kc, two_cb) &&
+            vqg_supported(0, pack_bits, dim, group, E, H, I, kc, false)) {
+            rc = launch_sort_rows(inds, P, 1, (int)E, vqg_tile_rows(0, dim), list, y, H, st, &sr);
+            if (rc) return rc;
+            uint16_t* x16 = (uint16_t*)((char*)list + sort_index_bytes(P, 4096, 1));
+            rc = launch_vqg_to_f16(x, T * H, x16, st);
+            if (rc) return rc;
+            VqgArgs g = {};
+            g.x = x16; g.xrows = T; g.lhs_div = k; g.tiles = sr.tiles; g.sorted = sr.sorted; g.E = E;
+            g.codes[0] = codes_gate; g.codes[1] = codes_up;
+            g.sc[0] = (const uint16_t*)scales_gate; g.sc[1] = (const uint16_t*)scales_up;
+            g.cb[0] = (const uint16_t*)codebook_gate; g.cb[1] = (const uint16_t*)codebook_up;
+            g.kc = kc; g.N = I; g.K = H; g.W = Wg; g.group = group; g.y = act; g.rows = P; g.y_f16 = 1;
+            rc = launch_vqg(g, 0, pack_bits, dim, true, sr.max_tiles, st);
+            if (rc) return rc;
+            KMI_CHECK_LAUNCH("vq_gemm(glu)");
+            VqgArgs d = g;
+            d.x = act; d.xrows = P; d.lhs_div = 1;
+            d.codes[0] = d.codes[1] = codes_down;
+            d.sc[0] = d.sc[1] = (const uint16_t*)scales_down;
+            d.cb[0] = d.cb[1] = (const uint16_t*)codebook_down;
+            d.N = H; d.K = I; d.W = Wd; d.y = y; d.y_f16 = 0;
+            rc = launch_vqg(d, 0, pack_bits, dim, false, sr.max_tiles, st);
+            if (rc) return rc;
+            KMI_CHECK_LAUNCH("vq_gemm(down)");
+            if (scores) return kmi_moe_combine(y, scores, dtype, T, k, H, out, stream);
+            return OK;
+        }
         if (!formed) {
             void* index_ws = list;
             // the sort zeroes y's rows of out-of-range experts (no tile holds them)
