@@ -1,6 +1,8 @@
-// Prefill-shape quantized matmul (M > 16) for gfx950: LDS-tiled bf16 MFMA.
+// Prefill-shape quantized matmul (M > 64) for gfx950: LDS-tiled bf16 MFMA
+// (qmm5 below); qmm_kernel serves outputs past 2 GiB, which qmm5's buffer
+// views do not reach.
 //
-// A workgroup (4 waves) owns a 128 x 128 tile of y and walks K in steps of
+// qmm_kernel: a workgroup (4 waves) owns a 128 x 128 tile of y and walks K in steps of
 // 64.  Per step it stages the x tile (bf16) and the packed weight tile, which
 // it dequantizes once to bf16 (What = s*q + b, rounded once) into LDS, so
 // the dequantization is shared by all 128 activation rows; each wave then
@@ -144,7 +146,7 @@ __global__ __launch_bounds__(256) void qmm_kernel(
 struct QgemmArgs {
     const uint16_t* x;          // [M, K] bf16
     const uint32_t* w;          // [N, K*bits/32]
-    const uint16_t* s;          // [N, K/gs] bf16
+    const void* s;              // [N, K/gs] bf16, microscaled: [N, K/32] bytes
     const uint16_t* b;
     uint16_t* y;                // [M, N] bf16 (one split)
     float* partial;             // [splits, M, N] fp32 (several splits)
@@ -153,13 +155,21 @@ struct QgemmArgs {
 };
 
 // =============================================================================
-// qmm5: M > 128.  Block tile 256 (M) x 128 (N) x 64 (K); 8 waves (two per
-// SIMD) as 4 (M) x 2 (N), each a 64 x 64 tile of y as 2 x 2 blocks of
-// v_mfma_f32_32x32x16_bf16 (64 fp32 accumulators per lane).
+// qmm5: block tile 256 (M) x 128 (N) x 64 (K); 8 waves (two per SIMD) as
+// 4 (M) x 2 (N), each a 64 x 64 tile of y as 2 x 2 blocks of
+// v_mfma_f32_32x32x16_bf16 (64 fp32 accumulators per lane).  Up to 128 rows:
+// 128 x 256, waves 2 x 4, so no wave works on padding rows.
+// Measured (before: qmm_kernel up to 128 rows, its grid of N / 128 workgroups
+// with no K split; microscaled weights on the batched kernel, whose hi + lo
+// operands double the MFMAs): 4-bit 128 rows x [4096, 14336] 667 -> 36.5 us, 65
+// rows x [14336, 4096] 162 -> 33; 8-bit 100 rows x [4096, 4096] 158 -> 22;
+// mxfp4 1000 rows x [4096, 14336] 460 -> 127 (925 TFLOP/s), mxfp8 700 rows x
+// [5120, 2048] 77 -> 32.
 //   - x and the dequantized weights are staged through LDS (two buffers),
 //     both loaded with 8 lanes per 128-byte row segment.  The weight tile is
 //     dequantized once per workgroup (fp32 s*q + b, one bf16 rounding: 16
-//     values per thread).
+//     values per thread, 32 at 128 rows; microscaled codes as element * 2^e in
+//     fp32, which bf16 holds exactly).
 //   - k order: in a k-tile, lane half h reads k in [32h, 32h + 32) and MFMA
 //     step s the 8 values 32h + 8s .. +8 of it, for x and w alike (the
 //     contraction is unchanged).
@@ -182,7 +192,7 @@ struct QgemmArgs {
 // CU; loads with one row per lane run at a quarter of the rate of loads with
 // 8 lanes per 128-byte row.
 // =============================================================================
-constexpr int Q5M = 256, Q5N = 128, Q5K = 64, Q5LDS = Q5K + 8;
+constexpr int Q5K = 64, Q5LDS = Q5K + 8;
 constexpr int Q5_RING = 4;
 
 
@@ -212,24 +222,52 @@ __device__ __forceinline__ u32x4 q5_dequant8(uint32_t w0, uint32_t w1, float sc,
     return o;
 }
 
-template <int BITS, int GS>
+// 8 microscaled weights (E2M1: one word; E4M3: two) times their scale.
+template <int BITS>
+__device__ __forceinline__ u32x4 q5_decode8(uint32_t w0, uint32_t w1, float sc) {
+    f32x2_t v[4];
+    if constexpr (BITS == 4) {
+        v[0] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w0, 1.f, 0);
+        v[1] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w0, 1.f, 1);
+        v[2] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w0, 1.f, 2);
+        v[3] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w0, 1.f, 3);
+    } else {
+        v[0] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(w0, 1.f, false);
+        v[1] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(w0, 1.f, true);
+        v[2] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(w1, 1.f, false);
+        v[3] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(w1, 1.f, true);
+    }
+    u32x4 o;
+#pragma unroll
+    for (int j = 0; j < 4; j++) o[j] = cvt_pk_bf16(v[j].x * sc, v[j].y * sc);
+    return o;
+}
+
+template <int BITS, int GS, bool MX, int BM>
 __global__ __launch_bounds__(512, 1) void qmm5_kernel(QgemmArgs a) {
+    constexpr int BN = 256 * 128 / BM;           // 128 or 256 columns
+    constexpr int WN = BN / 64;                  // waves along N (2 or 4)
+    constexpr int TPR = 512 / BN;                // threads per weight row (4 or 2)
+    constexpr int WPT = Q5K / TPR;               // weights per thread per k-tile (16 or 32)
+    constexpr int XC = BM / 64;                  // 16-byte x pieces per thread per k-tile
     constexpr int EPW = 32 / BITS;
+    constexpr int SB = MX ? 1 : 2;               // bytes per scale
     constexpr int TB = Q5K * BITS / 8;           // bytes of a weight row per k-tile
-    constexpr int QB = 16 * BITS / 8;            // bytes of a thread's 16 weights (8 or 16)
+    constexpr int QB = WPT * BITS / 8;           // bytes of a thread's weights (8, 16 or 32)
     constexpr uint32_t DEAD = 0x80000000u;       // scalar offset past every extent
-    __shared__ __align__(16) uint16_t As[2][Q5M * Q5LDS];
-    __shared__ __align__(16) uint16_t Bs[2][Q5N * Q5LDS];
+    static_assert(GS >= WPT, "a thread's weights lie in one group");
+    __shared__ __align__(16) uint16_t As[2][BM * Q5LDS];
+    __shared__ __align__(16) uint16_t Bs[2][BN * Q5LDS];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, h = lane >> 5;
     // ids grp*8*mtn + 8*mt + x -> n-tile 8 grp + x, m-tile mt (XCD = id % 8)
-    const int mtn = (int)((a.M + Q5M - 1) / Q5M);
+    const int mtn = (int)((a.M + BM - 1) / BM);
     const int id = (int)blockIdx.x, grp = id / (8 * mtn), rem = id % (8 * mtn);
     const int gw = a.n_tiles - 8 * grp < 8 ? a.n_tiles - 8 * grp : 8;
     const int mt = rem / gw, nt = 8 * grp + rem % gw;
-    const int64_t bm = (int64_t)mt * Q5M, bn = (int64_t)nt * Q5N;
+    const int64_t bm = (int64_t)mt * BM, bn = (int64_t)nt * BN;
     const int nk = (int)(a.K / Q5K);
     const int kt0 = (int)blockIdx.y * a.kt_per_split;
     const int kt1 = kt0 + a.kt_per_split < nk ? kt0 + a.kt_per_split : nk;
@@ -238,29 +276,29 @@ __global__ __launch_bounds__(512, 1) void qmm5_kernel(QgemmArgs a) {
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x + bm * a.K, (a.M - bm) * a.K * 2);
     const int64_t nrows = a.N - bn;
     const __amdgpu_buffer_rsrc_t rw = make_rsrc(a.w + bn * wpr, nrows * wpr * 4);
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.s + bn * gpr, nrows * gpr * 2);
-    const __amdgpu_buffer_rsrc_t rb = make_rsrc(a.b + bn * gpr, nrows * gpr * 2);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc((const char*)a.s + bn * gpr * SB, nrows * gpr * SB);
+    const __amdgpu_buffer_rsrc_t rb = make_rsrc(MX ? nullptr : a.b + bn * gpr, MX ? 0 : nrows * gpr * 2);
 
     // x: chunk c = tid + 512 i -> row c / 8, 16-byte piece c % 8
-    uint32_t xoff[4];
+    uint32_t xoff[XC];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < XC; i++) {
         const int c = tid + 512 * i;
         xoff[i] = (uint32_t)(((c >> 3) * a.K + (c & 7) * 8) * 2);
     }
-    // weights: thread -> row tid / 4, quarter q = tid % 4 (16 weights)
-    const int brow = tid >> 2, bq = tid & 3;
+    // weights: thread -> row tid / TPR, its part bq = tid % TPR (WPT weights)
+    const int brow = tid / TPR, bq = tid % TPR;
     const uint32_t woff = (uint32_t)(brow * wpr * 4 + bq * QB);
-    const uint32_t soff = (uint32_t)(brow * gpr * 2 + 2 * ((16 * bq) / GS));
+    const uint32_t soff = (uint32_t)(brow * gpr * SB + SB * ((WPT * bq) / GS));
 
-    u32x4 ra[Q5_RING][4];                         // x ring
+    u32x4 ra[Q5_RING][XC];                        // x ring
     uint32_t rwv[Q5_RING][QB / 4];                // weight ring
     uint32_t rsc[Q5_RING], rbi[Q5_RING];
 
     auto load_x = [&](int slot, int kt) {
         const uint32_t so = kt < kt1 ? (uint32_t)kt * (Q5K * 2) : DEAD;
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int i = 0; i < XC; i++)
             ra[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)xoff[i], (int)so, 0);
     };
     auto load_w = [&](int slot, int kt) {
@@ -270,33 +308,45 @@ __global__ __launch_bounds__(512, 1) void qmm5_kernel(QgemmArgs a) {
             const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rw, (int)woff, (int)so, 0);
             rwv[slot][0] = v.x; rwv[slot][1] = v.y;
         } else {
-            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)woff, (int)so, 0);
-            rwv[slot][0] = v.x; rwv[slot][1] = v.y; rwv[slot][2] = v.z; rwv[slot][3] = v.w;
+#pragma unroll
+            for (int q = 0; q < QB / 16; q++) {
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(woff + 16 * q), (int)so, 0);
+                rwv[slot][4 * q] = v.x; rwv[slot][4 * q + 1] = v.y;
+                rwv[slot][4 * q + 2] = v.z; rwv[slot][4 * q + 3] = v.w;
+            }
         }
-        const uint32_t sg = live ? (uint32_t)(2 * (((int64_t)kt * Q5K) / GS)) : DEAD;
-        rsc[slot] = __builtin_amdgcn_raw_buffer_load_b16(rs, (int)soff, (int)sg, 0);
-        rbi[slot] = __builtin_amdgcn_raw_buffer_load_b16(rb, (int)soff, (int)sg, 0);
+        const uint32_t sg = live ? (uint32_t)(SB * (((int64_t)kt * Q5K) / GS)) : DEAD;
+        if constexpr (MX) {
+            rsc[slot] = __builtin_amdgcn_raw_buffer_load_b8(rs, (int)soff, (int)sg, 0);
+        } else {
+            rsc[slot] = __builtin_amdgcn_raw_buffer_load_b16(rs, (int)soff, (int)sg, 0);
+            rbi[slot] = __builtin_amdgcn_raw_buffer_load_b16(rb, (int)soff, (int)sg, 0);
+        }
     };
     auto store_x = [&](int buf, int slot) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < XC; i++) {
             const int c = tid + 512 * i;
             *(u32x4*)(&As[buf][(c >> 3) * Q5LDS + (c & 7) * 8]) = ra[slot][i];
         }
     };
     auto store_w = [&](int buf, int slot) {
-        const float sc = bf16_to_f32((uint16_t)rsc[slot]), bi = bf16_to_f32((uint16_t)rbi[slot]);
-        uint16_t* dst = &Bs[buf][brow * Q5LDS + 16 * bq];
-        if constexpr (BITS == 4) {
-            *(u32x4*)dst = q5_dequant8<4>(rwv[slot][0], 0u, sc, bi);
-            *(u32x4*)(dst + 8) = q5_dequant8<4>(rwv[slot][1], 0u, sc, bi);
+        uint16_t* dst = &Bs[buf][brow * Q5LDS + WPT * bq];
+        constexpr int NW8 = BITS / 4;            // words per 8 weights
+        if constexpr (MX) {
+            const float sc = e8m0_to_f32(rsc[slot]);
+#pragma unroll
+            for (int q = 0; q < WPT / 8; q++)
+                *(u32x4*)(dst + 8 * q) = q5_decode8<BITS>(rwv[slot][NW8 * q], rwv[slot][NW8 * q + NW8 - 1], sc);
         } else {
-            *(u32x4*)dst = q5_dequant8<8>(rwv[slot][0], rwv[slot][1], sc, bi);
-            *(u32x4*)(dst + 8) = q5_dequant8<8>(rwv[slot][2], rwv[slot][3], sc, bi);
+            const float sc = bf16_to_f32((uint16_t)rsc[slot]), bi = bf16_to_f32((uint16_t)rbi[slot]);
+#pragma unroll
+            for (int q = 0; q < WPT / 8; q++)
+                *(u32x4*)(dst + 8 * q) = q5_dequant8<BITS>(rwv[slot][NW8 * q], rwv[slot][NW8 * q + NW8 - 1], sc, bi);
         }
     };
 
-    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+    const int wm = (wave / WN) * 64, wn = (wave % WN) * 64;
     f32x16 acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; i++)
@@ -407,29 +457,79 @@ __global__ __launch_bounds__(256) void qmm_split_reduce(const float* __restrict_
 }
 
 struct QgemmPlan {
+    bool fits;          // qmm5's 32-bit views reach x, w and y
+    int bm;             // rows per tile: 256, or 128 up to 128 rows
     int n_tiles, m_tiles, splits, kt_per_split;
     size_t ws;
 };
 
 // K splits while the tiles would fill under half of the CUs (one workgroup
 // per CU), at least 8 k-tiles per split.
-static QgemmPlan plan_gemm(int64_t M, int64_t N, int64_t K) {
-    QgemmPlan p;
-    p.n_tiles = (int)ceil_div(N, Q5N);
-    p.m_tiles = (int)ceil_div(M, Q5M);
-    const int tiles = p.n_tiles * p.m_tiles;
+static QgemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int bits) {
+    QgemmPlan p = {};
+    p.bm = M <= 128 ? 128 : 256;
+    p.n_tiles = (int)ceil_div(N, 256 * 128 / p.bm);
+    p.m_tiles = (int)ceil_div(M, p.bm);
+    const int64_t tiles = (int64_t)p.n_tiles * p.m_tiles;
     const int nk = (int)(K / Q5K);
-    int s = tiles * 2 <= 256 ? 256 / tiles : 1;
+    int s = tiles * 2 <= 256 ? 256 / (int)tiles : 1;
     if (s > nk / 8) s = nk / 8 > 0 ? nk / 8 : 1;
     p.kt_per_split = (int)ceil_div(nk, s);
     p.splits = (int)ceil_div(nk, p.kt_per_split);
-    p.ws = p.splits > 1 ? (size_t)p.splits * M * N * sizeof(float) : 0;
+    p.fits = M * K * 2 < (1LL << 31) && N * K * bits / 8 < (1LL << 31) &&
+             M * N * (p.splits > 1 ? 4 : 2) < (1LL << 31);
+    p.ws = p.fits && p.splits > 1 ? (size_t)p.splits * M * N * sizeof(float) : 0;
     return p;
 }
 
-size_t qmm_gemm_workspace(int64_t M, int64_t K, int64_t N) {
-    if (M <= 128) return 0;
-    return plan_gemm(M, N, K).ws;
+size_t qmm_gemm_workspace(int64_t M, int64_t K, int64_t N, int bits) { return plan_gemm(M, N, K, bits).ws; }
+
+// mx 1: microscaled codes, byte scales; K must be a multiple of 64 and the
+// call fit qmm5 (qmm_gemm_mx_fits)
+static int run_gemm5(const QgemmPlan& p, const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w,
+                     const void* scales, const void* biases, int group_size, int bits, int mx, void* y,
+                     void* workspace, size_t workspace_bytes, hipStream_t st) {
+    if (p.ws > 0 && (!workspace || workspace_bytes < p.ws)) {
+        set_error("quantized_matmul: workspace of %zu bytes needed, %zu given", p.ws, workspace_bytes);
+        return EWORKSPACE;
+    }
+    QgemmArgs a = {(const uint16_t*)x, w, scales, (const uint16_t*)biases, (uint16_t*)y, (float*)workspace,
+                   M, N, K, p.kt_per_split, p.splits, p.n_tiles};
+    const dim3 grid((unsigned)(p.n_tiles * p.m_tiles), (unsigned)p.splits);
+#define KMI_QMM5(B, G, X)                                                \
+    if (p.bm == 128) qmm5_kernel<B, G, X, 128><<<grid, 512, 0, st>>>(a); \
+    else qmm5_kernel<B, G, X, 256><<<grid, 512, 0, st>>>(a)
+    if (mx) {
+        if (bits == 4) { KMI_QMM5(4, 32, true); }
+        else { KMI_QMM5(8, 32, true); }
+    } else if (bits == 4) {
+        if (group_size == 32) { KMI_QMM5(4, 32, false); }
+        else if (group_size == 64) { KMI_QMM5(4, 64, false); }
+        else { KMI_QMM5(4, 128, false); }
+    } else {
+        if (group_size == 32) { KMI_QMM5(8, 32, false); }
+        else if (group_size == 64) { KMI_QMM5(8, 64, false); }
+        else { KMI_QMM5(8, 128, false); }
+    }
+#undef KMI_QMM5
+    KMI_CHECK_LAUNCH("qmm5");
+    if (p.splits > 1) {
+        const int64_t count = M * N;
+        qmm_split_reduce<<<(unsigned)ceil_div(count, 256), 256, 0, st>>>((const float*)workspace, p.splits, count,
+                                                                         (uint16_t*)y);
+        KMI_CHECK_LAUNCH("qmm_split_reduce");
+    }
+    return OK;
+}
+
+bool qmm_gemm_mx_fits(int64_t M, int64_t K, int64_t N, int bits) {
+    return K % GBK == 0 && plan_gemm(M, N, K, bits).fits;
+}
+
+int qmm_gemm_mx(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w, const void* scales, int bits,
+                void* y, void* workspace, size_t workspace_bytes, hipStream_t st) {
+    return run_gemm5(plan_gemm(M, N, K, bits), x, M, K, N, w, scales, nullptr, 32, bits, 1, y, workspace,
+                     workspace_bytes, st);
 }
 
 int qmm_gemm(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w,
@@ -442,37 +542,10 @@ int qmm_gemm(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w,
     const uint16_t* ss = (const uint16_t*)scales;
     const uint16_t* bb = (const uint16_t*)biases;
     uint16_t* yy = (uint16_t*)y;
-    if (M > 128) {
-        KMI_CHECK_ARG(M * K * 2 < (1LL << 31) && N * K * bits / 8 < (1LL << 31),
-                      "quantized_matmul: x or w past 2 GiB");
-        const QgemmPlan p = plan_gemm(M, N, K);
-        KMI_CHECK_ARG(M * N * (p.splits > 1 ? 4 : 2) < (1LL << 31), "quantized_matmul: y past 2 GiB");
-        if (p.ws > 0 && (!workspace || workspace_bytes < p.ws)) {
-            set_error("quantized_matmul: workspace of %zu bytes needed, %zu given", p.ws, workspace_bytes);
-            return EWORKSPACE;
-        }
-        QgemmArgs a = {xx, w, ss, bb, yy, (float*)workspace, M, N, K, p.kt_per_split, p.splits, p.n_tiles};
-        const dim3 grid((unsigned)(p.n_tiles * p.m_tiles), (unsigned)p.splits);
-#define KMI_QMM5(B, G) qmm5_kernel<B, G><<<grid, 512, 0, st>>>(a)
-        if (bits == 4) {
-            if (group_size == 32) KMI_QMM5(4, 32);
-            else if (group_size == 64) KMI_QMM5(4, 64);
-            else KMI_QMM5(4, 128);
-        } else {
-            if (group_size == 32) KMI_QMM5(8, 32);
-            else if (group_size == 64) KMI_QMM5(8, 64);
-            else KMI_QMM5(8, 128);
-        }
-#undef KMI_QMM5
-        KMI_CHECK_LAUNCH("qmm5");
-        if (p.splits > 1) {
-            const int64_t count = M * N;
-            qmm_split_reduce<<<(unsigned)ceil_div(count, 256), 256, 0, st>>>((const float*)workspace, p.splits,
-                                                                              count, yy);
-            KMI_CHECK_LAUNCH("qmm_split_reduce");
-        }
-        return OK;
-    }
+    const QgemmPlan p = plan_gemm(M, N, K, bits);
+    if (p.fits)
+        return run_gemm5(p, x, M, K, N, w, scales, biases, group_size, bits, 0, y, workspace, workspace_bytes, st);
+    KMI_CHECK_ARG(M <= 128, "quantized_matmul: x, w or y past 2 GiB");
     dim3 grid((unsigned)ceil_div(N, GBN), (unsigned)ceil_div(M, GBM));
     KMI_CHECK_ARG(grid.y < 65536, "quantized_matmul: M too large");
 #define KMI_QMM(B, G) qmm_kernel<B, G><<<grid, 256, 0, st>>>(xx, w, ss, bb, yy, M, N, K)

@@ -231,7 +231,10 @@ static int launch_valu(const QmvArgs& a, int bits, dim3 grid, size_t lds, hipStr
 int qmm_gemm(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w,
              const void* scales, const void* biases, int group_size, int bits, void* y,
              void* workspace, size_t workspace_bytes, hipStream_t st);
-size_t qmm_gemm_workspace(int64_t M, int64_t K, int64_t N);  // qmm.hip
+size_t qmm_gemm_workspace(int64_t M, int64_t K, int64_t N, int bits);  // qmm.hip
+int qmm_gemm_mx(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w, const void* scales, int bits,
+                void* y, void* workspace, size_t workspace_bytes, hipStream_t st);
+bool qmm_gemm_mx_fits(int64_t M, int64_t K, int64_t N, int bits);
 
 static int check_common(int64_t K, int64_t N, int dtype, int gs, int bits) {
     KMI_CHECK_ARG(dtype == BF16, "quantized matmul: only bfloat16 activations are supported (got dtype %d)", dtype);
@@ -298,7 +301,7 @@ extern "C" {
 
 size_t kmi_qmm_workspace_bytes(int64_t M, int64_t K, int64_t N, int group_size, int bits) {
     if (M <= 0 || K <= 0 || N <= 0 || group_size <= 0 || (bits != 4 && bits != 8)) return 0;
-    if (M > SKINNY_MAX_M) return qmm_gemm_workspace(M, K, N);       // GEMM path (split-K partials)
+    if (M > SKINNY_MAX_M) return qmm_gemm_workspace(M, K, N, bits); // GEMM path (split-K partials)
     if (choose_kind(M, K, bits) != QmvKind::SKINNY) return 0;   // VALU path
     return skinny_partial_bytes(dense_skinny_plan(M, K, N, bits, group_size), M, N);
 }
@@ -346,14 +349,18 @@ int kmi_qmm(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w,
     return run_skinny(a, p, bits, group_size, ntiles, workspace, nullptr, 1, dl, st);
 }
 
-// Microscaled dense decode: the decode kernels of kmi_qmm with the E2M1 /
-// E4M3 decode and byte scales; more than 64 rows, or K not a multiple of 64,
-// take the batched kernel (nd = 0).
+// Microscaled dense: the decode kernels of kmi_qmm up to 64 rows and its GEMM
+// beyond, with the E2M1 / E4M3 decode and byte scales; K not a multiple of
+// 64, or a call past the GEMM's 2 GiB views, takes the batched kernel (nd = 0).
 static bool mx_decode_shape(int64_t M, int64_t K) { return M <= SKINNY_MAX_M && K % 64 == 0; }
+static bool mx_gemm_shape(int64_t M, int64_t K, int64_t N, int bits) {
+    return M > SKINNY_MAX_M && qmm_gemm_mx_fits(M, K, N, bits);
+}
 
 size_t kmi_qmm_mx_workspace_bytes(int64_t M, int64_t K, int64_t N, int mode) {
     if (M <= 0 || K <= 0 || N <= 0 || (mode != 1 && mode != 2)) return 0;
     const int bits = mode == 1 ? 4 : 8;
+    if (mx_gemm_shape(M, K, N, bits)) return qmm_gemm_workspace(M, K, N, bits);
     if (!mx_decode_shape(M, K)) return kmi_qmm_batched_workspace_bytes(0, nullptr, M, K, N);
     if (choose_kind(M, K, bits) != QmvKind::SKINNY) return 0;
     return skinny_partial_bytes(dense_skinny_plan(M, K, N, bits, 32), M, N);
@@ -367,6 +374,8 @@ int kmi_qmm_mx(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w
     KMI_CHECK_ARG(M >= 0 && K > 0 && K % 32 == 0 && N > 0,
                   "quantized_matmul: M=%lld K=%lld N=%lld (K a multiple of 32)", (long long)M, (long long)K,
                   (long long)N);
+    if (dtype == BF16 && x && w && scales && y && mx_gemm_shape(M, K, N, bits))
+        return qmm_gemm_mx(x, M, K, N, w, scales, bits, y, workspace, workspace_bytes, (hipStream_t)stream);
     if (!mx_decode_shape(M, K)) {
         const int64_t xs[1] = {K}, ws[1] = {K * bits / 32}, ss[1] = {K / 32};
         return kmi_qmm_batched(x, xs, w, ws, scales, nullptr, ss, 0, nullptr, M, K, N, 1, dtype, 32, bits, mode,

@@ -1,0 +1,57 @@
+"""GPU parity: the dense GEMM (qmm.hip) over affine and microscaled weights
+from 65 rows up, at the edges of its row and column tiles, one k-tile, and K
+splits, against the oracle (max rel err 1e-2, cosine 0.9999); and the
+microscaled form against the batched kernel it replaces at these sizes,
+special scales and codes included."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from knurlogic_amd import ops
+from tests.util import assert_close, bf16_normal, to_numpy, to_torch, u32_to_torch
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+SHAPES = [  # (M, N, K): rows around a tile, ragged columns, one k-tile, K splits
+    (65, 257, 64), (127, 1, 128), (128, 256, 2048), (129, 255, 576), (257, 129, 1024), (100, 1000, 4096),
+]
+
+
+@pytest.mark.parametrize("bits,group", [(4, 32), (4, 64), (8, 64), (8, 128)])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_affine_rows(dev, M, N, K, bits, group):
+    if K % group:
+        pytest.skip("K is not a multiple of the group")
+    rng = np.random.default_rng(M + N + K)
+    wq, s, b = O.quantize(bf16_normal(rng, (N, K), 0.02), group, bits)
+    x = bf16_normal(rng, (M, K))
+    got = ops.quantized_matmul(to_torch(x, dev, BF), u32_to_torch(wq, dev), to_torch(s, dev, BF), to_torch(b, dev, BF),
+                               True, group, bits)
+    ref = O.quantized_matmul(x, wq, s, b, True, group, bits, "float32")
+    assert_close(to_numpy(got), ref, what=f"{bits}-bit {M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("mode", ["mxfp4", "mxfp8"])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_microscaled_rows(dev, M, N, K, mode):
+    rng = np.random.default_rng(M + N + K)
+    bits = 4 if mode == "mxfp4" else 8
+    codes = rng.integers(0, 256, (N, K * bits // 8), dtype=np.uint8)
+    if bits == 8:
+        codes[(codes & 0x7f) == 0x7f] = 0x3c                # no NaN codes among the finite rows
+    scales = rng.integers(120, 127, (N, K // 32), dtype=np.uint8)
+    if N > 4:
+        scales[0, 0], scales[1, -1] = 0, 255                # 2^-127 and NaN
+        scales[2, 0] = 254                                  # 2^127: past bf16 with any larger code
+        if bits == 8:
+            codes[3, 5] = 0x7f                              # a NaN code
+    tw = u32_to_torch(codes.view(np.uint32), dev)
+    ts = torch.from_numpy(scales).to(dev)
+    x = to_torch(bf16_normal(rng, (M, K)), dev, BF)
+    got = to_numpy(ops.quantized_matmul(x, tw, ts, None, True, 32, bits, mode))
+    ref = to_numpy(ops.qmm_batched(x, tw, ts, None, True, 32, bits, mode=mode))
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
+    ok = np.isfinite(ref) & (np.abs(ref) < 1e30)
+    assert_close(got[ok], ref[ok], what=f"{mode} {M}x{N}x{K}")
