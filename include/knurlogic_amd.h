@@ -293,6 +293,24 @@ int kmi_masked_softmax(const void* x, int64_t ldx, int dtype, const int64_t* row
                        void* stream);
 
 /*
+ * mlx-lm's quantized attention (.../_mlx_vlm/models/base.py:260-302) of a
+ * prompt chunk in one pass: q [B, H, L, D] bf16 contiguous (scaled by `scale`
+ * rounded to bf16, the product rounded) over K and V triples (codes, bf16
+ * scales and biases) of [B, Hk, N, *] at 4 or 8 bits, groups of 64, D = 64, 128
+ * or 256.  strides: element strides (b, h, n) of K's codes, scales, biases, then
+ * V's; code strides are multiples of 4 words from 16-byte aligned bases.  causal:
+ * key j hidden from query l when j > N - L + l (N >= L).  Scores are rounded to
+ * bf16 as the separate products round them; each probability times its key's
+ * scale is rounded to bf16 once.  `workspace` holds the key splits' fp32 sums
+ * (kmi_sdpa_prefill_workspace_bytes; may be NULL when that is 0).
+ */
+size_t kmi_sdpa_prefill_workspace_bytes(int64_t B, int64_t H, int64_t Hk, int64_t L, int64_t N, int64_t D);
+int kmi_sdpa_prefill(const void* q, int64_t B, int64_t H, int64_t L, int64_t D, const uint32_t* kw, const void* ks,
+                     const void* kb, const uint32_t* vw, const void* vs, const void* vb, const int64_t* strides,
+                     int64_t Hk, int64_t N, int group_size, int bits, float scale, int causal, void* out,
+                     void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * mlx's nn.Linear for the layers a quantized model keeps unquantized: the
  * Qwen3.5-MoE router gate and shared-expert gate (qwen3_5.py:173-174,186,
  * self.gate(x) / self.shared_expert_gate(x)):

@@ -38,6 +38,9 @@ SIGNATURES = {
     "kmi_qmm_batched": (I, [P, P, P, P, P, P, P, I, P, I64, I64, I64, I, I, I, I, I, P, P, I64, I64,
                             ctypes.c_float, P, I64, P, SZ, P]),
     "kmi_qmm_batched_workspace_bytes": (SZ, [I, P, I64, I64, I64]),
+    "kmi_sdpa_prefill_workspace_bytes": (SZ, [I64, I64, I64, I64, I64, I64]),
+    "kmi_sdpa_prefill": (I, [P, I64, I64, I64, I64, P, P, P, P, P, P, P, I64, I64, I, I, ctypes.c_float, I, P, P,
+                             SZ, P]),
     "kmi_masked_softmax": (I, [P, I64, I, P, I64, P, I, P, P, I64, P]),
     "kmi_vq_packed_gather_qmm": (I, [P, I64, I64, P, I, P, I, I, P, I, I64, I64, P, I64, P, I64, I, P, P]),
     "kmi_vq_packed_glu": (I, [P, I64, I64, I64, P, P, P, P, P, P, I, I, I, I, I64, P, I64, P, I64, I, P, P]),

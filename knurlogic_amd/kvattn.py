@@ -25,6 +25,7 @@ reference kernel's rule, :11-12), where a plain softmax would give NaN.
 """
 from __future__ import annotations
 
+import ctypes
 import logging
 import os
 import sys
@@ -242,6 +243,39 @@ def masked_softmax(scores, mask=None, out=None):
     return out
 
 
+#: query rows per KV head (rep x L) from which quantized_sdpa runs as one pass
+#: over the keys (kmi_sdpa_prefill's tiles hold 128)
+PREFILL_ROWS = 64
+
+
+def _prefill_strides(q, K, V, mask, group: int, bits: int):
+    """The 18 element strides kmi_sdpa_prefill takes, or None where the call
+    stays on the separate products: masks given as tensors, other widths,
+    groups or head dims, few query rows, layouts the kernel does not read."""
+    if not (mask is None or mask == "causal") or bits not in (4, 8) or group != 64:
+        return None
+    B, H, L, D = q.shape
+    if D not in (64, 128, 256) or q.dtype != torch.bfloat16 or not q.is_cuda:
+        return None
+    shape = tuple(K[0].shape[:-1])
+    if len(shape) != 3 or shape[0] != B or H // shape[1] * L < PREFILL_ROWS or shape[2] < (1 if mask is None else L):
+        return None
+    st = []
+    for w, s, b in (K, V):
+        if b is None or w.dtype not in (torch.uint32, torch.int32) or w.data_ptr() % 16 or not w.is_cuda:
+            return None
+        for t, cols in ((w, D * bits // 32), (s, D // 64), (b, D // 64)):
+            if tuple(t.shape) != shape + (cols,) or (cols > 1 and t.stride(3) != 1):
+                return None
+            if t is not w and (t.dtype != torch.bfloat16 or not t.is_cuda):
+                return None
+            one = [t.stride(i) if n > 1 else 0 for i, n in enumerate(shape)]
+            if t is w and any(x % 4 for x in one):
+                return None
+            st += one
+    return st
+
+
 def quantized_sdpa(queries, q_keys, q_values, scale: float, mask=None, group_size: int = 64,
                    bits: int = 8):
     """mlx-lm's quantized_scaled_dot_product_attention (.../_mlx_vlm/
@@ -250,14 +284,31 @@ def quantized_sdpa(queries, q_keys, q_values, scale: float, mask=None, group_siz
     dtype (mlx casts the scalar), the product rounded to bf16, scores =
     quantized_matmul(q, K, transpose=True) in bf16, masked, softmax(precise)
     in bf16, out = quantized_matmul(p, V, transpose=False).  GQA query heads
-    share their KV head's triple (broadcast, never copied).  Three HIP
-    launches (four when the keys are split across workgroups)."""
+    share their KV head's triple (broadcast, never copied).  A prompt chunk
+    over 4 or 8-bit groups of 64, unmasked or causal, runs as one pass over
+    the keys (kmi_sdpa_prefill, and a merge when the keys are split); other
+    calls as three HIP launches (four when the keys are split across
+    workgroups)."""
     B, Hq, L, D = queries.shape
     Hk = q_keys[0].shape[-3]
     if Hq % Hk:
         raise ValueError(f"quantized_sdpa: {Hq} query heads over {Hk} KV heads")
     rep = Hq // Hk
     q = queries
+    st = _prefill_strides(q, q_keys, q_values, mask, group_size, bits)
+    if st is not None:
+        q = q.contiguous()
+        if q.data_ptr() % 16:
+            q = q.clone()
+        N = q_keys[0].shape[-2]
+        out = torch.empty_like(q)
+        lib = _abi.load()
+        nbytes = lib.kmi_sdpa_prefill_workspace_bytes(B, Hq, Hk, L, N, D)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+        _abi.check(lib.kmi_sdpa_prefill(
+            _ptr(q), B, Hq, L, D, *(_ptr(t) for t in (*q_keys, *q_values)), (ctypes.c_int64 * 18)(*st), Hk, N, 64,
+            bits, float(scale), int(mask is not None), _ptr(out), _ptr(ws), nbytes, _stream(q)), "quantized_sdpa")
+        return out
     Kt, Vt = tuple(q_keys), tuple(q_values)
     if rep > 1:
         q = q.reshape(B, Hk, rep, L, D)

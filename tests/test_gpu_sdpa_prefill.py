@@ -1,0 +1,78 @@
+"""GPU parity: a prompt chunk's attention over the quantized cache in one pass
+(kmi_sdpa_prefill through kvattn.quantized_sdpa) against the oracle's mlx-lm
+quantized attention: tiles of 64 keys and 128 query rows and their remainders,
+key splits, causal chunks that start the cache, strided slab views, both code
+widths, keys far from zero (the group biases), and what stays on the separate
+products.  Bar: max rel err 1e-2, cosine 0.9999 (both sides round scores to
+bf16; each rounds a probability once)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from knurlogic_amd import kvattn
+from tests.util import assert_close, bf16_normal, to_numpy, to_torch, u32_to_torch
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+def _kv(rng, B, Hk, cap, D, bits, dev, mean=0.0):
+    w = O.bf16_round((rng.standard_normal((B, Hk, cap, D)) + mean).astype(np.float32))
+    wq, s, b = O.quantize(w, 64, bits)
+    return (wq, s, b), (u32_to_torch(wq, dev), to_torch(s, dev, BF), to_torch(b, dev, BF))
+
+
+@pytest.mark.parametrize("B,H,Hk,L,N,D,bits,mask", [
+    (1, 2, 1, 32, 32, 128, 8, "causal"),       # 64 rows, one half-filled tile of keys, every diagonal
+    (1, 4, 2, 65, 65, 128, 8, "causal"),       # rows past a tile, heads inside a row tile
+    (2, 4, 1, 40, 127, 64, 8, "causal"),
+    (1, 3, 3, 64, 129, 128, 4, None),
+    (1, 8, 2, 50, 700, 128, 8, "causal"),      # key splits
+    (1, 4, 1, 33, 1111, 256, 8, "causal"),
+    (1, 2, 2, 70, 300, 256, 4, "causal"),
+    (1, 2, 1, 200, 513, 64, 4, None),
+])
+def test_matches_the_oracle(dev, B, H, Hk, L, N, D, bits, mask):
+    rng = np.random.default_rng(L + N + D + bits)
+    cap = N + 19
+    K, tK = _kv(rng, B, Hk, cap, D, bits, dev, 0.5)
+    V, tV = _kv(rng, B, Hk, cap, D, bits, dev, -0.3)
+    view = lambda t: tuple(x[:, :, :N] for x in t)
+    q = bf16_normal(rng, (B, H, L, D))
+    tq = to_torch(q, dev, BF)
+    got = kvattn.quantized_sdpa(tq, view(tK), view(tV), D ** -0.5, mask, 64, bits)
+    assert kvattn._prefill_strides(tq, view(tK), view(tV), mask, 64, bits) is not None
+    ref = O.quantized_sdpa(q, view(K), view(V), D ** -0.5, mask, 64, bits)
+    assert_close(to_numpy(got), ref, what="one pass")
+    assert torch.equal(got, kvattn.quantized_sdpa(tq, view(tK), view(tV), D ** -0.5, mask, 64, bits))
+
+
+def test_slots_past_the_keys_are_not_read_into_the_result(dev):
+    """A slab's slots past N hold whatever was there: NaN scales and biases
+    in them leave the result alone."""
+    rng = np.random.default_rng(3)
+    K, tK = _kv(rng, 1, 2, 256, 128, 8, dev)
+    V, tV = _kv(rng, 1, 2, 256, 128, 8, dev)
+    q = to_torch(bf16_normal(rng, (1, 4, 64, 128)), dev, BF)
+    view = lambda t: tuple(x[:, :, :100] for x in t)
+    before = kvattn.quantized_sdpa(q, view(tK), view(tV), 0.088, "causal")
+    for t in (tK, tV):
+        t[1][:, :, 100:] = float("nan")
+        t[2][:, :, 100:] = float("nan")
+    assert torch.equal(before, kvattn.quantized_sdpa(q, view(tK), view(tV), 0.088, "causal"))
+
+
+def test_other_calls_keep_the_separate_products(dev):
+    rng = np.random.default_rng(4)
+    _, tK = _kv(rng, 1, 2, 96, 128, 8, dev)
+    q = to_torch(bf16_normal(rng, (1, 4, 64, 128)), dev, BF)
+    few = q[:, :, :4]
+    add = torch.zeros(64, 96, dtype=BF, device=dev)
+    short = tuple(t[:, :, :40] for t in tK)                   # causal rows that see no key
+    odd = (tK[0][:, :, :, ::1].transpose(2, 3).contiguous().transpose(2, 3), *tK[1:])
+    for qq, kk, mask, group in ((few, tK, "causal", 64), (q, tK, add, 64), (q, short, "causal", 64),
+                                (q, odd, None, 64), (q, tK, None, 32)):
+        assert kvattn._prefill_strides(qq, kk, kk, mask, group, 8) is None
+    out = kvattn.quantized_sdpa(q, tK, tK, 0.1, add)
+    assert_close(to_numpy(out), to_numpy(kvattn.quantized_sdpa(q, tK, tK, 0.1, None)), what="zero mask")
