@@ -30,6 +30,7 @@ static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 struct GluPlan {
     bool tok;
     bool gemm;      // expert tiles of 128 or 256 rows on the grouped GEMM (moe_gemm.hip)
+    bool eg;        // expert tiles of up to 160 rows (moe_eg.hip)
     int tm;
     size_t act, y, idx, total;
 };
@@ -37,10 +38,19 @@ struct GluPlan {
 // Rows per active expert from which both projections run as a grouped GEMM
 // (prefill chunks: 64 rows fill four 16-row fragments of the skinny kernels)
 constexpr int64_t GEMM_MIN_ROWS = 64;
+// From the same row count 4-bit experts take moe_eg's tiles where its gate/up
+// grid (one workgroup per expert tile and 256 output columns, one per CU)
+// fills half of the CUs: 128 experts 2048 -> 768 -> 2048, 2048 tokens 400 us on
+// moe_gemm, 285 here, 1024 tokens 269 vs 225; 60 experts 1920 -> 704, 2048
+// tokens 218 vs 144; but 32 experts 1536 -> 512 at 64 rows each (64 workgroups)
+// 70 vs 79.  Below GEMM_MIN_ROWS the skinny kernels stay also where they are
+// slower (512 tokens 296 vs 193): they hold the weights exactly, this kernel
+// rounds them to bf16 as moe_gemm does.
+constexpr int64_t EG_MIN_GRID = 128;
 
 // rows per tile: the average routed pairs per active expert, in 16-row chunks
-// (gemm_ok: the grouped GEMM takes these weights)
-static GluPlan plan_glu(int64_t T, int64_t H, int64_t I, int k, int64_t E, bool gemm_ok) {
+// (gemm_ok, eg_ok: the grouped GEMMs take these weights)
+static GluPlan plan_glu(int64_t T, int64_t H, int64_t I, int k, int64_t E, bool gemm_ok, bool eg_ok) {
     GluPlan p = {};
     const int64_t P = T * k;
     p.tok = P <= TOK_MAX_PAIRS;
@@ -52,11 +62,13 @@ static GluPlan plan_glu(int64_t T, int64_t H, int64_t I, int k, int64_t E, bool 
         // then stage their x rows once per workgroup (qgemv_xs) with two
         // workgroups per CU
         const int tm_skinny = rpt <= 2 ? 4 : qgemv_gather_tile_rows(rpt);
-        p.gemm = gemm_ok && rpt >= GEMM_MIN_ROWS;
-        p.tm = p.gemm ? (rpt <= 128 ? 128 : 256) : tm_skinny;
+        p.eg = eg_ok && rpt >= GEMM_MIN_ROWS &&
+               active * ceil_div(rpt, moe_eg_tile_rows()) * ceil_div(I, 256) >= EG_MIN_GRID;
+        p.gemm = !p.eg && gemm_ok && rpt >= GEMM_MIN_ROWS;
+        p.tm = p.eg ? moe_eg_tile_rows() : p.gemm ? (rpt <= 128 ? 128 : 256) : tm_skinny;
         p.y = align256((size_t)P * H * 2);
         // sized for either tiling, so the workspace query need not know the mode
-        const size_t a = sort_index_bytes(P, E, tm_skinny), b = sort_index_bytes(P, E, p.gemm ? p.tm : tm_skinny);
+        const size_t a = sort_index_bytes(P, E, tm_skinny), b = sort_index_bytes(P, E, p.tm);
         p.idx = a > b ? a : b;
     }
     p.total = p.act + p.y + p.idx;
@@ -72,7 +84,8 @@ extern "C" {
 size_t kmi_switch_glu_workspace_bytes(int64_t T, int64_t H, int64_t I, int k, int64_t E,
                                       int group_size, int bits) {
     if (T <= 0 || H <= 0 || I <= 0 || k <= 0 || E <= 0) return 0;
-    return plan_glu(T, H, I, k, E, moe_gemm_supported(H, I, bits, group_size, 0)).total;
+    return plan_glu(T, H, I, k, E, moe_gemm_supported(H, I, bits, group_size, 0),
+                    moe_eg_supported(H, I, bits, group_size, 0)).total;
 }
 
 }  // extern "C"
@@ -106,7 +119,8 @@ static int switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, int k
     KMI_CHECK_ARG(E <= 4096, "switch_glu: %lld experts (at most 4096)", (long long)E);
     KMI_CHECK_ARG(T * H * 2 < (1LL << 31) && T * k * (H > I ? H : I) * 2 < (1LL << 31),
                   "switch_glu: activations past 2 GiB");
-    const GluPlan p = plan_glu(T, H, I, k, E, moe_gemm_supported(H, I, bits, group_size, mx));
+    const GluPlan p = plan_glu(T, H, I, k, E, moe_gemm_supported(H, I, bits, group_size, mx),
+                               moe_eg_supported(H, I, bits, group_size, mx));
     KMI_CHECK_ARG(!mx || group_size == 32, "switch_glu (mx): group %d (32)", group_size);
     if (!workspace || workspace_bytes < p.total) {
         set_error("switch_glu: workspace of %zu bytes needed, %zu given", p.total, workspace_bytes);
@@ -153,7 +167,7 @@ static int switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, int k
         have_sort = true;
         return launch_sort_rows(inds, P, 1, (int)E, p.tm, ws + p.act + p.y, y, H, st, &sr);
     };
-    const bool formed = routed && !p.gemm && p.tm == 4 && pair_tiles_fit(P, E, p.tm);
+    const bool formed = routed && !p.gemm && !p.eg && p.tm == 4 && pair_tiles_fit(P, E, p.tm);
     int rc = formed ? OK : sort();
     if (rc) return rc;
     const int64_t max_tiles = sort_max_tiles(P, E, p.tm);
@@ -175,8 +189,9 @@ static int switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, int k
         g.sorted_out = list;
         g.tiles_out = list + P;
     }
-    if (p.gemm) {
-        rc = launch_moe_gemm(g, bits, group_size, true, p.tm, max_tiles, st);
+    if (p.gemm || p.eg) {
+        rc = p.eg ? launch_moe_eg(g, group_size, true, max_tiles, st)
+                  : launch_moe_gemm(g, bits, group_size, true, p.tm, max_tiles, st);
         if (rc) return rc;
     } else {
         const QgPlan pg = plan_qgemv_unsplit(I, H, max_tiles, p.tm, group_size);
@@ -187,7 +202,7 @@ static int switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, int k
             if (rc) return rc;
         }
     }
-    KMI_CHECK_LAUNCH(p.gemm ? "moe_gemm(gate|up)" : "qgemv(gate|up)");
+    KMI_CHECK_LAUNCH(p.eg ? "moe_eg(gate|up)" : p.gemm ? "moe_gemm(gate|up)" : "qgemv(gate|up)");
     QgArgs d = {};
     d.x = act; d.xrows = P; d.w = w_down; d.s = (const uint16_t*)s_down; d.b = (const uint16_t*)b_down;
     d.E = E; d.N = H; d.K = I; d.erows = H; d.y = y; d.rows = P; d.tm = p.tm; d.tiles = sr.tiles; d.mx = mx;
@@ -196,8 +211,9 @@ static int switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, int k
         d.sorted = list;
         d.tiles = list + P;
     }
-    if (p.gemm) {
-        rc = launch_moe_gemm(d, bits, group_size, false, p.tm, max_tiles, st);
+    if (p.gemm || p.eg) {
+        rc = p.eg ? launch_moe_eg(d, group_size, false, max_tiles, st)
+                  : launch_moe_gemm(d, bits, group_size, false, p.tm, max_tiles, st);
         if (rc) return rc;
     } else {
         const QgPlan pd = plan_qgemv_unsplit(H, I, max_tiles, p.tm, group_size);
@@ -210,7 +226,7 @@ static int switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, int k
             if (rc) return rc;
         }
     }
-    KMI_CHECK_LAUNCH(p.gemm ? "moe_gemm(down)" : "qgemv(down)");
+    KMI_CHECK_LAUNCH(p.eg ? "moe_eg(down)" : p.gemm ? "moe_gemm(down)" : "qgemv(down)");
     if (scores) return kmi_moe_combine(y, scores, dtype, T, k, H, out, stream);
     return OK;
 }
@@ -248,7 +264,7 @@ int kmi_moe_experts(const void* x, const void* logits, int64_t T, int64_t H, int
                   "moe_experts: top-%d of %lld experts (k <= 8, E <= %d)", k, (long long)E, ROUTE_MAX_E);
     if (T == 0) return OK;
     KMI_CHECK_ARG(logits && inds && scores, "moe_experts: null pointer");
-    const GluPlan p = plan_glu(T, H, I, k, E, false);
+    const GluPlan p = plan_glu(T, H, I, k, E, false, false);
     if (p.tok && E <= ROUTE_THREADS)   // decode sizes: the gate/up kernel routes its own token
         return switch_glu_impl(x, T, H, I, k, inds, scores, w_gu, s_gu, b_gu, w_down, s_down, b_down, E, dtype,
                                group_size, bits, out, workspace, workspace_bytes, stream, logits, inds, scores);

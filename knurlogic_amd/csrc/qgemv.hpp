@@ -81,6 +81,12 @@ bool moe_gemm_supported(int64_t H, int64_t I, int bits, int gs, int mx);
 int launch_moe_gemm(const QgArgs& a, int bits, int gs, bool glu, int tile_rows, int64_t tile_slots,
                     hipStream_t st);
 
+// The same over 4-bit weights (group 64 or 128, K % 64 == 0) in tiles of up to
+// moe_eg_tile_rows() rows whose cost follows their rows (moe_eg.hip).
+bool moe_eg_supported(int64_t H, int64_t I, int bits, int gs, int mx);
+int moe_eg_tile_rows();
+int launch_moe_eg(const QgArgs& a, int gs, bool glu, int64_t tile_slots, hipStream_t st);
+
 // glu: gate rows at 0, up rows at a.up_off, out = SwiGLU(gate, up) in bf16
 int launch_qgemv(const QgArgs& a, const QgPlan& p, int bits, int gs, bool glu, int64_t ntiles,
                  hipStream_t st);

@@ -112,3 +112,34 @@ def test_grouped_gemm_with_k_tiles_past_a_group(dev, bits):
     assert got.shape == (T, k, h) and np.isfinite(got).all()
     s = _sample(rng, T)
     assert_close(got[s], O.switch_glu(x[s], inds[s], *fns), what=f"grouped gemm {bits}-bit")
+
+
+@pytest.mark.parametrize("h,i_,group", [(320, 1984, 64), (256, 2048, 128), (64, 2048, 64)])
+def test_expert_tiles_at_their_edges(dev, h, i_, group):
+    """4-bit experts on tiles whose work follows their rows (moe_eg.hip):
+    row counts around its 32-row blocks and its largest tile, an expert
+    without rows, columns that do not fill a column block, one and several
+    K stages, pairs whose expert is out of range."""
+    rng = np.random.default_rng(9300 + h)
+    counts = [1, 31, 32, 33, 64, 65, 95, 127, 128, 129, 159, 160, 161, 330, 0, 40]
+    e = len(counts)
+    mats = []
+    for N, Kd in ((i_, h), (i_, h), (h, i_)):
+        wq = np.frombuffer(rng.bytes(e * N * Kd // 2), np.uint32).reshape(e, N, Kd // 8)
+        sc = O.bf16_round(rng.uniform(0.004, 0.008, (e, N, Kd // group)).astype(np.float32))
+        bi = O.bf16_round((-7.5 * sc + rng.normal(0, 0.002, sc.shape)).astype(np.float32))
+        mats.append((wq, sc, bi))
+    q = lambda m: nn.QuantizedSwitchLinear(u32_to_torch(m[0], dev), to_torch(m[1], dev, BF),
+                                           to_torch(m[2], dev, BF), None, group, 4)
+    glu = nn.SwitchGLU(*(q(m) for m in mats))
+    inds = np.concatenate([np.full(n, x) for x, n in enumerate(counts)] + [[e, -1]]).astype(np.int32)
+    rng.shuffle(inds)
+    x = bf16_normal(rng, (len(inds), h))
+    tx, ti = to_torch(x, dev, BF), torch.from_numpy(inds[:, None]).to(dev)
+    got = glu(tx, ti)
+    assert torch.equal(got, glu(tx, ti)), "a repeated call differs"
+    y, bad = to_numpy(got)[:, 0], (inds < 0) | (inds >= e)
+    assert (y[bad] == 0).all()
+    fns = [lambda xs, ex, m=m: O.quantized_matmul(xs, m[0][ex], m[1][ex], m[2][ex], True, group, 4, "bfloat16")
+           for m in mats]
+    assert_close(y[~bad], O.switch_glu(x[~bad], inds[~bad, None], *fns)[:, 0], what="expert tiles")
