@@ -41,8 +41,15 @@ __global__ __launch_bounds__(256) void qmv_reduce(const float* __restrict__ part
 // and never listed (the index arrays are not validated on the host).  Within
 // an expert the order of rows follows atomic arrival; each row's result does
 // not depend on its position.
+// One workgroup does it all, so up to SORT_REG single-row pairs per thread are
+// loaded at once and stay in registers with the place their count gave them
+// (one pass of atomics instead of two, no load inside the loops), and the list
+// is put together in LDS and written out in order (a store per row to its own
+// line took most of the time): 16384 pairs
+// 17.3 -> 11.0 us, 4096 8.0 -> 7.3.
 constexpr int SORT_THREADS = 1024;
 constexpr int SORT_MAX_E = 4096;
+constexpr int SORT_REG = 16;
 
 // Exclusive prefix sum over the workgroup's threads (thread order), and the
 // total in *total.  `wsum` holds SORT_THREADS / 64 ints of LDS.
@@ -82,12 +89,31 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_rows_by_expert(
     __shared__ int cursor[SORT_MAX_E];
     __shared__ int wsum[SORT_THREADS / 64];
     const int tid = threadIdx.x;
+    __shared__ uint16_t list[SORT_THREADS * SORT_REG];
+    const bool in_regs = Mper == 1 && P <= SORT_THREADS * SORT_REG;
+    int re[SORT_REG], rank[SORT_REG];              // this thread's pairs: expert, place among its rows
+    if (in_regs) {
+#pragma unroll
+        for (int i = 0; i < SORT_REG; i++) {
+            if ((int64_t)i * SORT_THREADS >= P) break;      // (the same for every thread)
+            const int64_t p = tid + (int64_t)i * SORT_THREADS;
+            re[i] = p < P ? rhs[p] : -1;
+        }
+    }
     for (int e = tid; e < E; e += SORT_THREADS) cnt[e] = 0;
     for (int t = tid; t < 3 * max_tiles; t += SORT_THREADS) tiles[t] = 0;
     __syncthreads();
-    for (int64_t p = tid; p < P; p += SORT_THREADS) {
-        const int e = rhs[p];
-        if (e >= 0 && e < E) atomicAdd(&cnt[e], (int)Mper);
+    if (in_regs) {
+#pragma unroll
+        for (int i = 0; i < SORT_REG; i++) {
+            if ((int64_t)i * SORT_THREADS >= P) break;
+            if (re[i] >= 0 && re[i] < E) rank[i] = atomicAdd(&cnt[re[i]], 1);
+        }
+    } else {
+        for (int64_t p = tid; p < P; p += SORT_THREADS) {
+            const int e = rhs[p];
+            if (e >= 0 && e < E) atomicAdd(&cnt[e], (int)Mper);
+        }
     }
     __syncthreads();
     // thread tid owns experts [EPT*tid, EPT*tid + EPT): row and tile offsets by scans
@@ -119,15 +145,30 @@ __global__ __launch_bounds__(SORT_THREADS) void sort_rows_by_expert(
     }
     if (tid == 0) offsets[E] = total_rows;
     __syncthreads();
-    for (int64_t p = tid; p < P; p += SORT_THREADS) {
-        const int e = rhs[p];
+    auto place = [&](int64_t p, int e, int pos) {
         if (e < 0 || e >= E) {
             if (y)
                 for (int64_t i = 0; i < Mper * N; i++) y[p * Mper * N + i] = 0;
-            continue;
+            return;
         }
-        const int pos = atomicAdd(&cursor[e], (int)Mper);
         for (int64_t m = 0; m < Mper; m++) sorted[pos + m] = (int32_t)(p * Mper + m);
+    };
+    if (in_regs) {
+#pragma unroll
+        for (int i = 0; i < SORT_REG; i++) {
+            const int64_t p = tid + (int64_t)i * SORT_THREADS;
+            if ((int64_t)i * SORT_THREADS >= P) break;
+            if (p >= P) continue;
+            if (re[i] >= 0 && re[i] < E) list[cursor[re[i]] + rank[i]] = (uint16_t)p;
+            else place(p, re[i], 0);
+        }
+        __syncthreads();
+        for (int i = tid; i < total_rows; i += SORT_THREADS) sorted[i] = list[i];
+        return;
+    }
+    for (int64_t p = tid; p < P; p += SORT_THREADS) {
+        const int e = rhs[p];
+        place(p, e, e >= 0 && e < E ? atomicAdd(&cursor[e], (int)Mper) : 0);
     }
 }
 
