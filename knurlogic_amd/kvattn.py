@@ -44,6 +44,9 @@ _LOGGED: set = set()
 #: query rows per KV head (GQA ratio x query length) the kernel takes
 MAX_ROWS = 64
 
+#: (b, h, n) element strides of K's codes, scales and biases, then V's
+_STRIDES = ctypes.c_int64 * 18
+
 #: the kernel's on/off switch, the reference's knob (engine/kvattn.py:69):
 #: unset or any other value is on
 ENV = "KNURLOGIC_KV_KERNEL"
@@ -157,20 +160,20 @@ def decode_sdpa(q, K, V, scale: float, mask=None, group: int = 64, bits: int = 8
     N = K[0].shape[2]
     q = q.contiguous()
     out = torch.empty_like(q)
-    m = _mask_rows(mask, B, L, N, q.device)
+    m = None if mask is None else _mask_rows(mask, B, L, N, q.device)
     causal = 1 if (isinstance(mask, str) and mask == "causal" and L > 1) else 0
-    strides = []
-    for t in (*K, *V):
-        strides += [t.stride(0), t.stride(1), t.stride(2)]
-    st = torch.tensor(strides, dtype=torch.int64)      # host array, read by the launcher
+    kv = (*K, *V)
+    # host array, read by the launcher
+    st = _STRIDES(*[s for t in kv for s in t.stride()[:3]])
     L_ = _abi.load()
     nbytes = L_.kmi_kv8_workspace_bytes(B, H, Hk, L, N, D)
     ws = torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=q.device)
-    _abi.check(L_.kmi_kv8_decode(
-        _ptr(q), DTYPE_CODE[q.dtype], B, H, L, D,
-        _ptr(K[0]), _ptr(K[1]), _ptr(K[2]), _ptr(V[0]), _ptr(V[1]), _ptr(V[2]),
-        st.data_ptr(), DTYPE_CODE[K[1].dtype], Hk, N, group, float(scale),
-        _ptr(m), causal, _ptr(out), _ptr(ws), nbytes, _stream(q)), "kv8_decode")
+    rc = L_.kmi_kv8_decode(
+        q.data_ptr(), DTYPE_CODE[q.dtype], B, H, L, D, *[t.data_ptr() for t in kv],
+        st, DTYPE_CODE[K[1].dtype], Hk, N, group, float(scale),
+        _ptr(m), causal, out.data_ptr(), ws.data_ptr(), nbytes, _stream(q))
+    if rc:
+        _abi.check(rc, "kv8_decode")
     return out
 
 
@@ -306,7 +309,7 @@ def quantized_sdpa(queries, q_keys, q_values, scale: float, mask=None, group_siz
         nbytes = lib.kmi_sdpa_prefill_workspace_bytes(B, Hq, Hk, L, N, D)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
         _abi.check(lib.kmi_sdpa_prefill(
-            _ptr(q), B, Hq, L, D, *(_ptr(t) for t in (*q_keys, *q_values)), (ctypes.c_int64 * 18)(*st), Hk, N, 64,
+            _ptr(q), B, Hq, L, D, *(_ptr(t) for t in (*q_keys, *q_values)), _STRIDES(*st), Hk, N, 64,
             bits, float(scale), int(mask is not None), _ptr(out), _ptr(ws), nbytes, _stream(q)), "quantized_sdpa")
         return out
     Kt, Vt = tuple(q_keys), tuple(q_values)

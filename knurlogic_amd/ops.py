@@ -19,6 +19,9 @@ from . import _abi
 
 DTYPE_CODE = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
+
 #: dequantize rounding: T(T(s*q) + b) (mlx's op-by-op order) or T(fma(s, q, b))
 ROUND_OP_BY_OP = 0
 ROUND_FUSED = 1
@@ -36,7 +39,9 @@ def _on_gpu(*ts):
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the current stream's handle without building a Stream object (1.8 us of
+    # a small call's host time)
+    return _raw_stream(t.get_device())
 
 
 def _ptr(t):
@@ -235,11 +240,11 @@ def _check_affine_operands(x, w, scales, biases, group_size, bits, what):
     if x.dtype != torch.bfloat16:
         raise ValueError(f"{what}: only bfloat16 activations are implemented (got {x.dtype})")
     K = x.shape[-1]
-    if w.shape[-1] * 32 // bits != K:
+    wshape, sshape = w.shape, scales.shape
+    if wshape[-1] * 32 // bits != K:
         raise ValueError(f"{what}: x has {K} features but w packs "
-                         f"{w.shape[-1] * 32 // bits} at {bits} bits")
-    if scales.shape[-1] * group_size != K or scales.shape != biases.shape \
-            or scales.shape[:-1] != w.shape[:-1]:
+                         f"{wshape[-1] * 32 // bits} at {bits} bits")
+    if sshape[-1] * group_size != K or sshape != biases.shape or sshape[:-1] != wshape[:-1]:
         raise ValueError(f"{what}: scales {tuple(scales.shape)} / biases "
                          f"{tuple(biases.shape)} do not match w {tuple(w.shape)} "
                          f"at group {group_size}")
@@ -262,20 +267,22 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor,
     if not transpose or w.ndim != 2 or bits not in (4, 8) or mode != "affine":
         return qmm_batched(x, w, scales, biases, transpose, group_size, bits, mode=mode)
     _check_affine_operands(x, w, scales, biases, group_size, bits, "quantized_matmul")
-    K = x.shape[-1]
+    shape = x.shape
+    K = shape[-1]
     N = w.shape[0]
     x2 = x.contiguous()
     M = x2.numel() // K if K else 0
-    y = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
+    y = x.new_empty((*shape[:-1], N))
     L = _lib()
     nbytes = L.kmi_qmm_workspace_bytes(M, K, N, group_size, bits)
-    ws = _workspace(nbytes, x.device)
+    ws = _workspace(nbytes, x.device) if nbytes else None
     # contiguous copies held in locals until the call returns: a temporary
     # freed mid-call could hand its memory to the next copy
     wc, sc, bc = w.contiguous(), scales.contiguous(), biases.contiguous()
-    _abi.check(L.kmi_qmm(_ptr(x2), M, K, N, _ptr(wc), _ptr(sc), _ptr(bc), DTYPE_CODE[x.dtype],
-                         group_size, bits, _ptr(y), _ptr(ws), nbytes, _stream(x)),
-               "quantized_matmul")
+    rc = L.kmi_qmm(x2.data_ptr(), M, K, N, wc.data_ptr(), sc.data_ptr(), bc.data_ptr(), 0, group_size, bits,
+                   y.data_ptr(), _ptr(ws), nbytes, _stream(x))
+    if rc:
+        _abi.check(rc, "quantized_matmul")
     return y
 
 
