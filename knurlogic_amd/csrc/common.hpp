@@ -184,6 +184,16 @@ __device__ __forceinline__ uint32_t bytes_to_bf16x2(uint32_t w, int lo_byte) {
     return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
 
+// The 8 nibbles of a word as two words of bytes: the even codes and the odd
+// ones, for v_cvt_f32_ubyte0..3.  (Opaque to the compiler, which otherwise
+// folds the mask into a v_bfe_u32 per code ahead of each conversion.)
+__device__ __forceinline__ void nibble_bytes(uint32_t w, uint32_t& even, uint32_t& odd) {
+    even = w & 0x0F0F0F0Fu;
+    odd = (w >> 4) & 0x0F0F0F0Fu;
+    asm("" : "+v"(even));
+    asm("" : "+v"(odd));
+}
+
 // 4-bit nibbles -> bf16 "128 + q" pairs.  Register r holds nibbles r (low
 // half) and r+4 (high half) of the word: k order [0,4,1,5,2,6,3,7].
 __device__ __forceinline__ u32x4 nibbles_to_bf16_magic(uint32_t w) {

@@ -57,8 +57,10 @@ constexpr int eg_max_ring() {
     for (int nb = 1; nb <= EG_MAX_NB; nb++) m = eg_ring(nb) > m ? eg_ring(nb) : m;
     return m;
 }
-// a wave's scales or biases of 32 rows, in whole 1 KB loads
-__host__ __device__ constexpr int eg_sc_bytes(int G) { return (64 * G + 1023) / 1024 * 1024; }
+// a wave's scales or biases of 32 rows, in whole 1 KB loads: 16-byte pieces of
+// 8 groups, piece-major (row l's at 16 l: a stage's reads of 32 rows fall on
+// distinct banks; row-major they cost a fifth of the kernel)
+__host__ __device__ constexpr int eg_sc_bytes(int G) { return ((G + 7) / 8 * 512 + 1023) / 1024 * 1024; }
 
 template <int GS, bool GLU, int NB>
 __device__ __forceinline__ void eg_body(const QgArgs& a, int expert, int nt, unsigned char* smem, const int32_t* rid_s) {
@@ -111,11 +113,16 @@ __device__ __forceinline__ void eg_body(const QgArgs& a, int expert, int nt, uns
         for (int j = 0; j < 2; j++) eg_dma16(rw, dst + j * 1024, coff[j], so);
     };
     issue_c(0);
-    // scales and biases of block j's 32 rows: consecutive in memory
+    // scales and biases of block j's 32 rows.  Rows of an odd number of groups
+    // start between words, where 16-byte loads may not: their 32 rows are
+    // loaded as they lie in memory
+    const bool odd = G & 1;
+    const int scrow = odd ? 2 * G : 16, scpiece = odd ? 16 : 512;
 #pragma unroll
     for (int j = 0; j < 2; j++)
         for (int q = 0; q < scb; q += 1024) {
-            const int64_t off = row0[j] * G * 2 + q + 16 * lane;
+            const int u = q / 16 + lane;
+            const int64_t off = row0[j] * G * 2 + (odd ? 16 * u : (u % 32) * G * 2 + (u / 32) * 16);
             const uint32_t v = row0[j] < a.erows ? (uint32_t)off : EG_NONE;
             eg_dma16(rs, sw + (2 * j) * scb + q, v, 0);
             eg_dma16(rb, sw + (2 * j + 1) * scb + q, v, 0);
@@ -141,17 +148,18 @@ __device__ __forceinline__ void eg_body(const QgArgs& a, int expert, int nt, uns
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             c.w[j] = *(const u32x4*)(src + j * 1024 + lane * 16);
-            c.s[j] = bf16_to_f32(*(const uint16_t*)(sw + (2 * j) * scb + (l32 * G + g) * 2));
-            c.b[j] = bf16_to_f32(*(const uint16_t*)(sw + (2 * j + 1) * scb + (l32 * G + g) * 2));
+            const unsigned char* p = sw + (2 * j) * scb + l32 * scrow + (g >> 3) * scpiece + (g & 7) * 2;
+            c.s[j] = bf16_to_f32(*(const uint16_t*)p);
+            c.b[j] = bf16_to_f32(*(const uint16_t*)(p + scb));
         }
         return c;
     };
-    // weights 2 d, 2 d + 1 of step s, block j
-    auto piece = [&](const Stage& c, int j, int s, int d) -> uint32_t {
-        const uint32_t w = c.w[j][s];
-        const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
-        return cvt_pk_bf16(__builtin_fmaf(c.s[j], (float)((lo >> (8 * d)) & 0xffu), c.b[j]),
-                           __builtin_fmaf(c.s[j], (float)((hi >> (8 * d)) & 0xffu), c.b[j]));
+    // weights 2 d, 2 d + 1 of block j's word, split into bytes
+    uint32_t ev[2], od[2];
+    auto split = [&](const Stage& c, int j, int s) { nibble_bytes(c.w[j][s], ev[j], od[j]); };
+    auto piece = [&](const Stage& c, int j, int d) -> uint32_t {
+        return cvt_pk_bf16(__builtin_fmaf(c.s[j], (float)((ev[j] >> (8 * d)) & 0xffu), c.b[j]),
+                           __builtin_fmaf(c.s[j], (float)((od[j] >> (8 * d)) & 0xffu), c.b[j]));
     };
     // x fragment of row block i, step s: row 32 i + l32, piece 4 h + s
     uint32_t aoff[4];
@@ -173,9 +181,11 @@ __device__ __forceinline__ void eg_body(const QgArgs& a, int expert, int nt, uns
     Stage cw = read_stage(0);
     u32x4 B[2][2];                                  // [step parity][block]
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int j = 0; j < 2; j++) {
+        split(cw, j, 0);
 #pragma unroll
-        for (int d = 0; d < 4; d++) B[0][j][d] = piece(cw, j, 0, d);
+        for (int d = 0; d < 4; d++) B[0][j][d] = piece(cw, j, d);
+    }
     for (int t = 0; t < nk; t++) {
         eg_wait<PER*(S - 2)>();                     // this wave's x of stage t and codes of t + 1 are in LDS
         lds_barrier();                              // and every wave's x
@@ -200,8 +210,11 @@ __device__ __forceinline__ void eg_body(const QgArgs& a, int expert, int nt, uns
                 acc[i][j] = eg_mfma(A[q % 4], B[c][j], acc[i][j]);
 #pragma unroll
                 for (int p = 0; p < 8; p++)
-                    if (p * 2 * NB / 8 == 2 * i + j)
-                        B[c ^ 1][p / 4][p % 4] = s < 3 ? piece(cw, p / 4, s + 1, p % 4) : piece(cn, p / 4, 0, p % 4);
+                    if (p * 2 * NB / 8 == 2 * i + j) {
+                        const Stage& from = s < 3 ? cw : cn;
+                        if (p % 4 == 0) split(from, p / 4, (s + 1) % 4);
+                        B[c ^ 1][p / 4][p % 4] = piece(from, p / 4, p % 4);
+                    }
             }
             __builtin_amdgcn_sched_barrier(0);
         }

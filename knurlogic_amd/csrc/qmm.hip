@@ -206,10 +206,12 @@ template <int BITS>
 __device__ __forceinline__ u32x4 q5_dequant8(uint32_t w0, uint32_t w1, float sc, float bi) {
     u32x4 o;
     if constexpr (BITS == 4) {
+        uint32_t even, odd;
+        nibble_bytes(w0, even, odd);
 #pragma unroll
         for (int j = 0; j < 4; j++)
-            o[j] = cvt_pk_bf16(__builtin_fmaf(sc, (float)((w0 >> (8 * j)) & 15u), bi),
-                               __builtin_fmaf(sc, (float)((w0 >> (8 * j + 4)) & 15u), bi));
+            o[j] = cvt_pk_bf16(__builtin_fmaf(sc, (float)((even >> (8 * j)) & 255u), bi),
+                               __builtin_fmaf(sc, (float)((odd >> (8 * j)) & 255u), bi));
     } else {
 #pragma unroll
         for (int j = 0; j < 2; j++) {
