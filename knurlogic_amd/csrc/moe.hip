@@ -114,17 +114,17 @@ __global__ __launch_bounds__(64) void moe_combine_bf16x8(const uint16_t* __restr
                 if (s0 + j >= k) break;
                 const uint32_t w[4] = {v[j].x, v[j].y, v[j].z, v[j].w};   // scalars before any bit reinterpretation
 #pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const float yv = __uint_as_float(e % 2 ? w[e / 2] & 0xffff0000u : w[e / 2] << 16);
-                    acc[e] += (double)TBF16::round(yv * sc[j]);
+                for (int e = 0; e < 4; e++) {
+                    const uint32_t p = cvt_pk_bf16(__uint_as_float(w[e] << 16) * sc[j],
+                                                   __uint_as_float(w[e] & 0xffff0000u) * sc[j]);
+                    acc[2 * e] += (double)__uint_as_float(p << 16);
+                    acc[2 * e + 1] += (double)__uint_as_float(p & 0xffff0000u);
                 }
             }
         }
         uint32_t o[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-            o[e] = (uint32_t)f32_to_bf16(f64_to_f32(acc[2 * e])) |
-                   ((uint32_t)f32_to_bf16(f64_to_f32(acc[2 * e + 1])) << 16);
+        for (int e = 0; e < 4; e++) o[e] = cvt_pk_bf16(f64_to_f32(acc[2 * e]), f64_to_f32(acc[2 * e + 1]));
         *(u32x4*)(out + t * H + c * 8) = u32x4{o[0], o[1], o[2], o[3]};
     }
 }

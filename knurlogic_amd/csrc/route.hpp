@@ -139,7 +139,7 @@ __device__ __forceinline__ void route_from(const float (&x)[PER], int E, int k, 
     for (int j = 0; j < PER; j++) rank[j] = 0;
     // unrolled, so the broadcast LDS reads of several steps are in flight
     // together (a step per LDS round trip would take microseconds)
-    const int Ep = (E + 15) & ~15;
+    const int Ep = (tid & ~63) < E ? (E + 15) & ~15 : 0;   // (a wave past the experts has none to rank)
     for (int i = 0; i < Ep; i += 16) {
         uint64_t a[16];
 #pragma unroll
