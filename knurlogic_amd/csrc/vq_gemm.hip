@@ -87,14 +87,14 @@ struct VqgFmt {
     static constexpr int RL = PACKED ? (RUN + (PB == 16 ? 0 : 31) + 127) / 128 : 0;
     // direct-to-LDS loads of a wave per stage, and the LDS they fill: one-byte
     // codes 4 bytes per (row, half), 16-bit codes 16 bytes per row (two halves),
-    // packed RL x 16 bytes per (row, half) and its scale's word
-    static constexpr int LOADS = CB == 1 ? 2 : CB == 2 ? 1 : 2 * RL + 2;
-    static constexpr int BYTES = CB == 1 ? 512 : CB == 2 ? 1024 : 2 * (RL * 1024 + 256);
+    // packed RL x 16 bytes per (row, half)
+    static constexpr int LOADS = CB == 1 ? 2 : CB == 2 ? 1 : 2 * RL;
+    static constexpr int BYTES = CB == 1 ? 512 : CB == 2 ? 1024 : 2 * RL * 1024;
     // stages in the ring by row blocks: as deep as the codebooks leave LDS for
     static constexpr int stages(int nb) {
         if (CB == 1) return nb <= 4 ? 4 : 3;
         if (CB == 2) return nb <= 2 ? 4 : nb <= 4 ? 3 : 2;
-        return DIM == 2 || nb > 3 ? 2 : 3;
+        return DIM == 2 || nb > 2 ? 2 : 3;
     }
     // gathers a whole stage ahead, into a second operand set, where the
     // registers allow it
@@ -111,6 +111,11 @@ struct VqgFmt {
     }
 };
 
+// Packed: a wave's scales of 32 rows (two blocks of them), loaded once in whole
+// 1 KB loads: 16-byte pieces of 8 groups, piece-major (row l's at 16 l), so a
+// stage's reads of 32 rows fall on distinct banks
+__host__ __device__ constexpr int vqg_sc_bytes(int G) { return ((G + 7) / 8 * 512 + 1023) / 1024 * 1024; }
+
 struct VqgTile {
     int expert, count, nt;
 };
@@ -126,7 +131,11 @@ __device__ __forceinline__ void vqg_body(const VqgArgs& a, const VqgTile& tl, un
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, h = lane >> 5;
     const int K = (int)a.K, nk = K / VQG_BK;
-    unsigned char* ar = smem + cbstride * (two_cb ? 2 : 1);
+    const int G = F::PACKED ? K / a.group : 0;
+    const int scb = F::PACKED ? vqg_sc_bytes(G) : 0;
+    unsigned char* sw = smem + cbstride * (two_cb ? 2 : 1);
+    unsigned char* ar = sw + VQG_WAVES * 2 * scb;
+    sw += wave * 2 * scb;                                    // this wave's scales
     unsigned char* cr = ar + S * AB + wave * F::BYTES;       // this wave's codes, S slots apart by 8 waves
 
     // x: load j of wave w fills rows 8 (w + 8 j) .. + 7
@@ -145,10 +154,9 @@ __device__ __forceinline__ void vqg_body(const VqgArgs& a, const VqgTile& tl, un
     for (int j = 0; j < 2; j++)
         col[j] = GLU ? tl.nt * 256 + 32 * wave + l32 : tl.nt * 512 + 64 * wave + 32 * j + l32;
     const int64_t e0 = (int64_t)tl.expert * a.N;
-    const int G = F::PACKED ? K / a.group : 1;
     const int gshift = F::PACKED && a.group == 128 ? 1 : 0;
-    __amdgpu_buffer_rsrc_t rc[2], rs[2];
-    uint32_t coff[2], soff[2];
+    __amdgpu_buffer_rsrc_t rc[2];
+    uint32_t coff[2];
 #pragma unroll
     for (int j = 0; j < 2; j++) {
         const int s = GLU ? j : 0;
@@ -158,10 +166,6 @@ __device__ __forceinline__ void vqg_body(const VqgArgs& a, const VqgTile& tl, un
         if constexpr (CB == 1) coff[j] = (uint32_t)(n * rb) + 4u * h;
         else coff[j] = (uint32_t)(n * a.W);                              // in words
         if constexpr (CB == 2) coff[j] = 0;
-        if constexpr (F::PACKED) {
-            rs[j] = make_rsrc(a.sc[s], a.E * a.N * G * 2);
-            soff[j] = (uint32_t)((e0 + n) * G);                          // in scales
-        }
     }
     // 16-bit codes: lane r moves the 16 bytes (both halves) of the wave's row r
     const unsigned char* cptr = nullptr;
@@ -196,12 +200,27 @@ __device__ __forceinline__ void vqg_body(const VqgArgs& a, const VqgTile& tl, un
 #pragma unroll
                 for (int q = 0; q < F::RL; q++)
                     vqg_dma16(rc[j], dst + (j * F::RL + q) * 1024, (coff[j] + w0 + 4u * q) * 4u, 0);
-                vqg_dma4(rs[j], dst + 2 * F::RL * 1024 + j * 256, ((soff[j] + (uint32_t)(t >> gshift)) * 2u) & ~3u, 0);
             }
         }
     };
 
     issue_c(0);
+    // Rows of an odd number of groups start between words, where 16-byte loads
+    // may not: their 32 rows are loaded as they lie in memory
+    const bool odd = G & 1;
+    const int scrow = odd ? 2 * G : 16, scpiece = odd ? 16 : 512;
+    if constexpr (F::PACKED) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.sc[GLU ? j : 0] + e0 * G, a.N * G * 2);
+            const int64_t row0 = col[j] - l32;
+            for (int q = 0; q < scb; q += 1024) {
+                const int u = q / 16 + lane;
+                const int64_t off = row0 * G * 2 + (odd ? 16 * u : (u % 32) * G * 2 + (u / 32) * 16);
+                vqg_dma16(rs, sw + j * scb + q, row0 < a.N ? (uint32_t)off : VQG_NONE, 0);
+            }
+        }
+    }
 #pragma unroll
     for (int t = 0; t < S - 1; t++) {
         issue_x(t);
@@ -243,6 +262,7 @@ __device__ __forceinline__ void vqg_body(const VqgArgs& a, const VqgTile& tl, un
     };
     auto read_codes = [&](int t) -> Codes {
         Codes c = {};
+        const int g = (t < nk ? t : nk - 1) >> gshift;
         const unsigned char* src = cr + (t % S) * (VQG_WAVES * F::BYTES);
 #pragma unroll
         for (int j = 0; j < 2; j++) {
@@ -256,12 +276,12 @@ __device__ __forceinline__ void vqg_body(const VqgArgs& a, const VqgTile& tl, un
                     const u32x4 v = *(const u32x4*)(src + (j * F::RL + q) * 1024 + lane * 16);
                     c.w[j][4 * q] = v.x; c.w[j][4 * q + 1] = v.y; c.w[j][4 * q + 2] = v.z; c.w[j][4 * q + 3] = v.w;
                 }
-                c.sc[j] = *(const uint32_t*)(src + 2 * F::RL * 1024 + j * 256 + lane * 4);
+                c.sc[j] = *(const uint16_t*)(sw + j * scb + l32 * scrow + (g >> 3) * scpiece + (g & 7) * 2);
             }
         }
         return c;
     };
-    // packed: bring a run to bit 0 and pick its scale
+    // packed: bring a run to bit 0
     auto settle = [&](Codes& c, int t0) {
         if constexpr (F::PACKED) {
             const int t = t0 < nk ? t0 : nk - 1;
@@ -273,7 +293,6 @@ __device__ __forceinline__ void vqg_body(const VqgArgs& a, const VqgTile& tl, un
                     for (int q = 0; q < 4 * F::RL - 1; q++)
                         c.w[j][q] = __builtin_amdgcn_alignbit(c.w[j][q + 1], c.w[j][q], sh);
                 }
-                c.sc[j] = ((soff[j] + (uint32_t)(t >> gshift)) & 1u) ? c.sc[j] >> 16 : c.sc[j] & 0xffffu;
             }
         }
     };
@@ -578,8 +597,9 @@ __global__ __launch_bounds__(256) void vqg_to_f16_kernel(const u32x4* __restrict
 
 int vqg_cbstride(int kc, int dim) { return (kc * dim * 2 + 15) & ~15; }
 
-size_t vqg_lds(int ring, int kc, int dim, bool two_cb) {
-    return (size_t)ring + (size_t)vqg_cbstride(kc, dim) * (two_cb ? 2 : 1);
+// G: scale groups per row (packed; else 0)
+size_t vqg_lds(int ring, int kc, int dim, bool two_cb, int G) {
+    return (size_t)ring + (size_t)vqg_cbstride(kc, dim) * (two_cb ? 2 : 1) + VQG_WAVES * 2 * vqg_sc_bytes(G);
 }
 
 // the packed layouts compiled: f(PB, DIM)
@@ -599,7 +619,7 @@ int vqg_ring(int code_bytes, int pack_bits, int dim) {
 template <int CB, int PB, int DIM>
 int vqg_go(const VqgArgs& a, bool glu, int64_t tile_slots, hipStream_t st) {
     const bool two_cb = glu && a.cb[1] != a.cb[0];
-    const size_t lds = vqg_lds(VqgFmt<CB, PB, DIM>::max_ring(), a.kc, DIM, two_cb);
+    const size_t lds = vqg_lds(VqgFmt<CB, PB, DIM>::max_ring(), a.kc, DIM, two_cb, CB ? 0 : (int)(a.K / a.group));
     const int n_tiles = (int)ceil_div(a.N, glu ? 256 : 512);
     const int64_t wgs = 8 * n_tiles * ceil_div(tile_slots, 8);
     if (wgs >= (1LL << 31)) {
@@ -626,11 +646,10 @@ bool vqg_supported(int code_bytes, int pack_bits, int dim, int group, int64_t E,
     if (code_bytes) {
         if (K % 128) return false;
     } else {
-        // scales are read as aligned words of two
-        if (!(group == 64 || group == 128) || K % group || (E * N * (K / group)) % 2) return false;
-        if (E * N * (K / group) * 2 >= (1LL << 31)) return false;
+        // an expert's scales start on a word
+        if (!(group == 64 || group == 128) || K % group || (N * (K / group)) % 2) return false;
     }
-    return vqg_lds(ring, kc, dim, two_cb) + VQG_RIDS * 4 <= 160 * 1024;
+    return vqg_lds(ring, kc, dim, two_cb, code_bytes ? 0 : (int)(K / group)) + VQG_RIDS * 4 <= 160 * 1024;
 }
 
 int launch_vqg(const VqgArgs& a, int code_bytes, int pack_bits, int dim, bool glu, int64_t tile_slots,

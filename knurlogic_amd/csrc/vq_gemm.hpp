@@ -26,7 +26,7 @@ struct VqgArgs {
 };
 
 // 32-row blocks of the largest tile the kernel takes, and its rows
-constexpr int vqg_max_blocks(int code_bytes, int dim) { return code_bytes ? 5 : dim == 2 ? 3 : 4; }
+constexpr int vqg_max_blocks(int code_bytes, int dim) { return code_bytes ? 5 : dim == 2 ? 2 : 4; }
 constexpr int vqg_tile_rows(int code_bytes, int dim) { return 32 * vqg_max_blocks(code_bytes, dim); }
 
 // Whether P routed pairs, avg rows per routed expert, run on this kernel
