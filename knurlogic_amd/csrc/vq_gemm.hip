@@ -98,7 +98,7 @@ struct VqgFmt {
     }
     // gathers a whole stage ahead, into a second operand set, where the
     // registers allow it
-    static constexpr bool ahead(int nb) { return stages(nb) >= 3 && nb <= (PACKED ? 1 : 4); }
+    static constexpr bool ahead(int nb) { return stages(nb) >= 3 && nb <= (PACKED ? 2 : 4); }
     static constexpr int a_bytes(int nb) { return (nb + 1) / 2 * 8192; }
     static constexpr int ring(int nb) { return stages(nb) * (a_bytes(nb) + VQG_WAVES * BYTES); }
     // row blocks of the largest tile: as many as the registers hold (packed
