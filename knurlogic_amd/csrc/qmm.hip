@@ -467,14 +467,14 @@ struct QgemmPlan {
 
 // K splits while the tiles would fill under half of the CUs (one workgroup
 // per CU), at least 8 k-tiles per split.
-static QgemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int bits) {
+static QgemmPlan plan_gemm(int64_t M, int64_t N, int64_t K, int bits, bool split = true) {
     QgemmPlan p = {};
     p.bm = M <= 128 ? 128 : 256;
     p.n_tiles = (int)ceil_div(N, 256 * 128 / p.bm);
     p.m_tiles = (int)ceil_div(M, p.bm);
     const int64_t tiles = (int64_t)p.n_tiles * p.m_tiles;
     const int nk = (int)(K / Q5K);
-    int s = tiles * 2 <= 256 ? 256 / (int)tiles : 1;
+    int s = split && tiles * 2 <= 256 ? 256 / (int)tiles : 1;
     if (s > nk / 8) s = nk / 8 > 0 ? nk / 8 : 1;
     p.kt_per_split = (int)ceil_div(nk, s);
     p.splits = (int)ceil_div(nk, p.kt_per_split);
@@ -530,8 +530,9 @@ bool qmm_gemm_mx_fits(int64_t M, int64_t K, int64_t N, int bits) {
 
 int qmm_gemm_mx(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w, const void* scales, int bits,
                 void* y, void* workspace, size_t workspace_bytes, hipStream_t st) {
-    return run_gemm5(plan_gemm(M, N, K, bits), x, M, K, N, w, scales, nullptr, 32, bits, 1, y, workspace,
-                     workspace_bytes, st);
+    QgemmPlan p = plan_gemm(M, N, K, bits);
+    if (p.ws > 0 && (!workspace || workspace_bytes < p.ws)) p = plan_gemm(M, N, K, bits, false);
+    return run_gemm5(p, x, M, K, N, w, scales, nullptr, 32, bits, 1, y, workspace, workspace_bytes, st);
 }
 
 int qmm_gemm(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w,
@@ -544,7 +545,9 @@ int qmm_gemm(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w,
     const uint16_t* ss = (const uint16_t*)scales;
     const uint16_t* bb = (const uint16_t*)biases;
     uint16_t* yy = (uint16_t*)y;
-    const QgemmPlan p = plan_gemm(M, N, K, bits);
+    QgemmPlan p = plan_gemm(M, N, K, bits);
+    // up to 128 rows a call without scratch runs unsplit
+    if (M <= 128 && p.ws > 0 && (!workspace || workspace_bytes < p.ws)) p = plan_gemm(M, N, K, bits, false);
     if (p.fits)
         return run_gemm5(p, x, M, K, N, w, scales, biases, group_size, bits, 0, y, workspace, workspace_bytes, st);
     KMI_CHECK_ARG(M <= 128, "quantized_matmul: x, w or y past 2 GiB");

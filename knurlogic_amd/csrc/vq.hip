@@ -431,10 +431,14 @@ int kmi_vq_glu(const void* x, int64_t T, int64_t H, int64_t I, int k, const int3
 static size_t vq_act_bytes(int64_t T, int64_t I, int k) { return ((size_t)T * k * I * 2 + 255) & ~(size_t)255; }
 static size_t vq_y_bytes(int64_t T, int64_t H, int k) { return ((size_t)T * k * H * 2 + 255) & ~(size_t)255; }
 
+// (what the calls that do not take the grouped GEMM need)
+static size_t vq_base_bytes(int64_t T, int64_t H, int64_t I, int k) {
+    return vq_act_bytes(T, I, k) + vq_y_bytes(T, H, k) + sort_index_bytes(T * k, 4096, 1);   // any tile size
+}
+
 size_t kmi_vq_switch_glu_workspace_bytes(int64_t T, int64_t H, int64_t I, int k) {
     if (T <= 0 || H <= 0 || I <= 0 || k <= 0) return 0;
-    return vq_act_bytes(T, I, k) + vq_y_bytes(T, H, k) + sort_index_bytes(T * k, 4096, 1) +   // any tile size
-           (size_t)T * H * 2;
+    return vq_base_bytes(T, H, I, k) + (size_t)T * H * 2;
 }
 
 }  // extern "C"
@@ -464,7 +468,7 @@ static int vq_switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, in
     KMI_CHECK_ARG(x && inds && codes_gate && scales_gate && codebook_gate && codes_up && scales_up &&
                   codebook_up && codes_down && scales_down && codebook_down && out,
                   "vq_switch_glu: null pointer");
-    const size_t need = kmi_vq_switch_glu_workspace_bytes(T, H, I, k);
+    const size_t need = vq_base_bytes(T, H, I, k);
     if (!workspace || workspace_bytes < need) {
         set_error("vq_switch_glu: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
         return EWORKSPACE;
@@ -499,10 +503,10 @@ static int vq_switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, in
     const bool formed = routed && !pair_mode && pair_tiles_fit(P, E, tile_rows);
     // Prefill: rows grouped by expert in large tiles on the codebook GEMM
     // (not where the router's call would form its tiles, so both calls agree)
-    const bool gemm = sortable && !pair_tiles_fit(P, E, tile_rows) && !pair_mode &&
-                      vqg_wanted(code_bytes, 8, P, avg) && al16(x) && al16(codes_gate) &&
-                      al16(codes_up) && al16(codes_down) && T * H * 2 < (1LL << 31) &&
-                      P * (H > I ? H : I) * 2 < (1LL << 31) &&
+    const bool gemm = m_glu && m_down && !pair_tiles_fit(P, E, tile_rows) && !pair_mode &&
+                      vqg_wanted(code_bytes, 8, P, avg) && al16(x) &&
+                      workspace_bytes >= kmi_vq_switch_glu_workspace_bytes(T, H, I, k) &&
+                      T * H * 2 < (1LL << 31) && P * (H > I ? H : I) * 2 < (1LL << 31) &&
                       vqg_supported(code_bytes, 0, 8, 0, E, I, H, kc, two_cb) &&
                       vqg_supported(code_bytes, 0, 8, 0, E, H, I, kc, false);
     SortedRows sr = {};

@@ -654,10 +654,14 @@ int kmi_vq_packed_glu(const void* x, int64_t X, int64_t H, int64_t I, const uint
 static size_t vps_act_bytes(int64_t P, int64_t I) { return ((size_t)P * I * 2 + 255) & ~(size_t)255; }
 static size_t vps_y_bytes(int64_t P, int64_t H) { return ((size_t)P * H * 2 + 255) & ~(size_t)255; }
 
+// (what the calls that do not take the grouped GEMM need)
+static size_t vps_base_bytes(int64_t P, int64_t H, int64_t I) {
+    return vps_act_bytes(P, I) + vps_y_bytes(P, H) + sort_index_bytes(P, 4096, 1);
+}
+
 size_t kmi_vq_packed_switch_glu_workspace_bytes(int64_t T, int64_t H, int64_t I, int k) {
     if (T <= 0 || H <= 0 || I <= 0 || k <= 0) return 0;
-    const int64_t P = T * k;
-    return vps_act_bytes(P, I) + vps_y_bytes(P, H) + sort_index_bytes(P, 4096, 1) + (size_t)T * H * 2;
+    return vps_base_bytes(T * k, H, I) + (size_t)T * H * 2;
 }
 
 }  // extern "C"
@@ -701,7 +705,7 @@ static int vps_switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, i
     const int64_t P = T * k;
     KMI_CHECK_ARG(P < 65536 && T * H * 2 < (1LL << 31) && P * (H > I ? H : I) * 2 < (1LL << 31),
                   "vq_packed_switch_glu: %lld (token, slot) pairs (at most 65535)", (long long)P);
-    const size_t need = kmi_vq_packed_switch_glu_workspace_bytes(T, H, I, k);
+    const size_t need = vps_base_bytes(P, H, I);
     if (!workspace || workspace_bytes < need) {
         set_error("vq_packed_switch_glu: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
         return EWORKSPACE;
@@ -733,6 +737,7 @@ static int vps_switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, i
         // Prefill: large expert tiles on the codebook GEMM (not where the
         // router's call would form its tiles, so both calls agree)
         if (!pair_tiles_fit(P, E, tile_rows) && vqg_wanted(0, dim, P, avg) && ((uintptr_t)x & 15u) == 0 &&
+            workspace_bytes >= kmi_vq_packed_switch_glu_workspace_bytes(T, H, I, k) &&
             (((uintptr_t)scales_gate | (uintptr_t)scales_up | (uintptr_t)scales_down) & 3u) == 0 &&
             I * Wg * 4 < (1LL << 31) && H * Wd * 4 < (1LL << 31) &&
             vqg_supported(0, pack_bits, dim, group, E, I, H, kc, two_cb) &&

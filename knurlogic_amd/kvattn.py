@@ -255,7 +255,7 @@ def _prefill_strides(q, K, V, mask, group: int, bits: int):
     """The 18 element strides kmi_sdpa_prefill takes, or None where the call
     stays on the separate products: masks given as tensors, other widths,
     groups or head dims, few query rows, layouts the kernel does not read."""
-    if not (mask is None or mask == "causal") or bits not in (4, 8) or group != 64:
+    if not (mask is None or (isinstance(mask, str) and mask == "causal")) or bits not in (4, 8) or group != 64:
         return None
     B, H, L, D = q.shape
     if D not in (64, 128, 256) or q.dtype != torch.bfloat16 or not q.is_cuda:

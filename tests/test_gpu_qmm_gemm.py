@@ -55,3 +55,31 @@ def test_microscaled_rows(dev, M, N, K, mode):
     assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
     ok = np.isfinite(ref) & (np.abs(ref) < 1e30)
     assert_close(got[ok], ref[ok], what=f"{mode} {M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("mode", ["affine", "mxfp4"])
+def test_up_to_128_rows_without_scratch(dev, mode):
+    """A C caller that passes no workspace where the plan would split K gets
+    the same product unsplit."""
+    from knurlogic_amd import _abi
+    rng = np.random.default_rng(5)
+    M, N, K = 100, 300, 2048
+    lib = _abi.load()
+    x = to_torch(bf16_normal(rng, (M, K)), dev, BF)
+    y = torch.empty(M, N, dtype=BF, device=dev)
+    wq, s, b = O.quantize(bf16_normal(rng, (N, K), 0.02), 64, 4)
+    w = u32_to_torch(wq, dev)
+    st = torch.cuda.current_stream().cuda_stream
+    if mode == "affine":
+        ts, tb = to_torch(s, dev, BF), to_torch(b, dev, BF)
+        assert lib.kmi_qmm_workspace_bytes(M, K, N, 64, 4) > 0
+        rc = lib.kmi_qmm(x.data_ptr(), M, K, N, w.data_ptr(), ts.data_ptr(), tb.data_ptr(), 0, 64, 4, y.data_ptr(),
+                         None, 0, st)
+        ref = ops.quantized_matmul(x, w, ts, tb, True, 64, 4)
+    else:
+        ts = torch.full((N, K // 32), 120, dtype=torch.uint8, device=dev)
+        assert lib.kmi_qmm_mx_workspace_bytes(M, K, N, 1) > 0
+        rc = lib.kmi_qmm_mx(x.data_ptr(), M, K, N, w.data_ptr(), ts.data_ptr(), 0, 1, y.data_ptr(), None, 0, st)
+        ref = ops.quantized_matmul(x, w, ts, None, True, 32, 4, "mxfp4")
+    assert rc == 0
+    assert_close(to_numpy(y), to_numpy(ref), what="no scratch")

@@ -40,8 +40,8 @@ def _check(rng, dev, glu, fns, counts, H):
     assert_close(comb[~bad], O.combine(ref[:, None], to_numpy(scores)[~bad]), what="vq gemm combine")
 
 
-@pytest.mark.parametrize("kc,shared,H,I", [(256, True, 256, 384), (256, False, 512, 128), (200, False, 128, 640),
-                                           (4096, True, 256, 384), (1024, False, 640, 128)])
+@pytest.mark.parametrize("kc,shared,H,I", [(256, True, 512, 768), (256, False, 768, 512), (200, False, 1024, 512),
+                                           (4096, True, 512, 768), (1024, False, 1024, 512)])
 def test_per_channel_scales(dev, kc, shared, H, I):
     rng = np.random.default_rng(kc + H + I)
     counts = [1, 31, 33, 160, 161, 650]
