@@ -41,7 +41,7 @@ constexpr int64_t GEMM_MIN_ROWS = 64;
 // From the same row count 4-bit experts take moe_eg's tiles where its gate/up
 // grid (one workgroup per expert tile and 256 output columns, one per CU)
 // fills half of the CUs: 128 experts 2048 -> 768 -> 2048, 2048 tokens 400 us on
-// moe_gemm, 285 here, 1024 tokens 269 vs 225; 60 experts 1920 -> 704, 2048
+// moe_gemm, 262 here, 1024 tokens 269 vs 225; 60 experts 1920 -> 704, 2048
 // tokens 218 vs 144; but 32 experts 1536 -> 512 at 64 rows each (64 workgroups)
 // 70 vs 79.  Below GEMM_MIN_ROWS the skinny kernels stay also where they are
 // slower (512 tokens 296 vs 193): they hold the weights exactly, this kernel

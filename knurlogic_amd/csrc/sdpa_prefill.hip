@@ -26,11 +26,11 @@
 // Few rows leave CUs idle: the keys are then split, each split writing fp32
 // sums with its maximum, merged by sdpa_merge.
 // Measured, 512 queries x 32 heads over 4 KV heads, 8192 8-bit keys, D = 128: the
-// separate products 515 us (233 scores, 152 softmax, 257 P V), one pass 150
-// (sdpa_prefill 143: vector instructions are issued 67% of the time, matrix
+// separate products 515 us (233 scores, 152 softmax, 257 P V), one pass 130
+// (vector instructions are issued 67% of the time, matrix
 // cores busy 25%); 120 queries over 882 keys 122 -> 26 us (one launch's host
-// work instead of three).  D = 256 holds one workgroup per CU: 400 queries over
-// 4000 keys 194 either way, 216 over 395 keys 115 -> 57.
+// work instead of three).  D = 256 holds one workgroup per CU: 512 queries x 16
+// heads over 2 KV heads, 4096 keys 229 -> 128, 300 over 2000 120 -> 107.
 #include "qgemv_dl.hpp"
 #include "../../include/knurlogic_amd.h"
 
