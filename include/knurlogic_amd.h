@@ -131,10 +131,10 @@ int kmi_dequantize_affine(const uint32_t* wq, const void* scales, const void* bi
  * src/knurlogic/engine/matmul_padding.py:94-105):
  *   y[M, N] = x[M, K] @ What[N, K]^T,  What = scale * q + bias,
  * fp32 accumulation, y rounded once to `dtype`.  x, scales, biases, y share
- * `dtype`.  Decode shapes (M <= 16) run the streaming GEMV kernel, larger M
- * the LDS-tiled MFMA GEMM.  Each output row depends only on its own input row.
+ * `dtype`.  Up to 64 rows run the streaming GEMV kernels, larger M the
+ * LDS-tiled MFMA GEMM.  Each output row depends only on its own input row.
  * `workspace` (kmi_qmm_workspace_bytes) holds split-K partials; it may be
- * NULL when that size is 0.
+ * NULL when that size is 0, or at 65..128 rows (K is then not split).
  */
 int kmi_qmm(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w,
             const void* scales, const void* biases, int dtype, int group_size,
@@ -152,7 +152,8 @@ size_t kmi_qmm_workspace_bytes(int64_t M, int64_t K, int64_t N, int group_size, 
  * biases; fp32 accumulation, y rounded once to bf16 (x and y bf16).  Up to
  * 64 rows with K a multiple of 64 run kmi_qmm's decode kernels (M = 1: the
  * streaming GEMV; 2..16 rows with K a multiple of 256: the direct-to-LDS
- * MFMA kernel; else the MFMA GEMV), anything else kmi_qmm_batched.  Each
+ * MFMA kernel; else the MFMA GEMV), more rows kmi_qmm's MFMA GEMM (x 16-byte
+ * aligned), anything else kmi_qmm_batched.  Each
  * output row depends only on its own input row.  `workspace`
  * (kmi_qmm_mx_workspace_bytes) holds split-K partials; it may be NULL when
  * that size is 0.
