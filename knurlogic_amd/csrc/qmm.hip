@@ -1,6 +1,6 @@
 // Prefill-shape quantized matmul (M > 64) for gfx950: LDS-tiled bf16 MFMA
-// (qmm5 below); qmm_kernel serves outputs past 2 GiB, which qmm5's buffer
-// views do not reach.
+// (qmm5 below); up to 128 rows qmm_kernel serves outputs past 2 GiB, which
+// qmm5's buffer views do not reach, and x off 16 bytes.
 //
 // qmm_kernel: a workgroup (4 waves) owns a 128 x 128 tile of y and walks K in steps of
 // 64.  Per step it stages the x tile (bf16) and the packed weight tile, which
@@ -548,9 +548,10 @@ int qmm_gemm(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w,
     QgemmPlan p = plan_gemm(M, N, K, bits);
     // up to 128 rows a call without scratch runs unsplit
     if (M <= 128 && p.ws > 0 && (!workspace || workspace_bytes < p.ws)) p = plan_gemm(M, N, K, bits, false);
-    if (p.fits)
+    // (x off 16 bytes stays on qmm_kernel there)
+    if (p.fits && (M > 128 || ((uintptr_t)x & 15u) == 0))
         return run_gemm5(p, x, M, K, N, w, scales, biases, group_size, bits, 0, y, workspace, workspace_bytes, st);
-    KMI_CHECK_ARG(M <= 128, "quantized_matmul: x, w or y past 2 GiB");
+    KMI_CHECK_ARG(p.fits || M <= 128, "quantized_matmul: x, w or y past 2 GiB");
     dim3 grid((unsigned)ceil_div(N, GBN), (unsigned)ceil_div(M, GBM));
     KMI_CHECK_ARG(grid.y < 65536, "quantized_matmul: M too large");
 #define KMI_QMM(B, G) qmm_kernel<B, G><<<grid, 256, 0, st>>>(xx, w, ss, bb, yy, M, N, K)
