@@ -20,7 +20,8 @@
 //     key's scale in fp32 and rounded once to bf16 (the reference rounds the
 //     probability); V's codes, centred on 2^(bits - 1), are exact in bf16; the
 //     biases' part of the sum is one fp32 dot product per query and group.
-//     The running maximum moves only when a step passes it by 8.
+//     A row's running maximum moves only when a step passes it by 8 (a row
+//     the step leaves alone is rescaled by 1).
 // A tile's K codes and V^T codes are decoded to LDS once for all 128 rows
 // (two buffers; the next tile's loads are in flight while a tile computes).
 // Few rows leave CUs idle: the keys are then split, each split writing fp32
@@ -338,7 +339,8 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void sdpa_prefill_kernel(SpAr
             for (int r = 1; r < 16; r++) mx = __builtin_fmaxf(mx, S[r]);
             mx = __builtin_fmaxf(mx, __shfl_xor(mx, 32, 64));
             if (__any(mx > m + 8.0f)) {
-                const float mn = mx > m ? mx : m;
+                // per row: what a row's neighbours score does not move its maximum
+                const float mn = mx > m + 8.0f ? mx : m;
                 const float f = __builtin_amdgcn_exp2f((m - mn) * SP_LOG2E);
                 m = mn;
                 lsum *= f;

@@ -76,3 +76,19 @@ def test_other_calls_keep_the_separate_products(dev):
         assert kvattn._prefill_strides(qq, kk, kk, mask, group, 8) is None
     out = kvattn.quantized_sdpa(q, tK, tK, 0.1, add)
     assert_close(to_numpy(out), to_numpy(kvattn.quantized_sdpa(q, tK, tK, 0.1, None)), what="zero mask")
+
+
+def test_a_row_does_not_depend_on_its_neighbours(dev):
+    """One query row made 40 times larger moves that row's maximum past 8
+    again and again; every other row stays what it was, bit for bit."""
+    rng = np.random.default_rng(11)
+    _, tK = _kv(rng, 1, 2, 1300, 128, 8, dev)
+    _, tV = _kv(rng, 1, 2, 1300, 128, 8, dev)
+    q = to_torch(bf16_normal(rng, (1, 4, 70, 128)), dev, BF)
+    other = q.clone()
+    other[0, 1, 37] *= 40
+    got, ref = (kvattn.quantized_sdpa(t, tK, tV, 128 ** -0.5, "causal") for t in (other, q))
+    same = torch.ones(1, 4, 70, dtype=torch.bool, device=dev)
+    same[0, 1, 37] = False
+    assert torch.equal(got[same], ref[same])
+    assert not torch.equal(got[~same], ref[~same])
