@@ -266,7 +266,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void sdpa_prefill_kernel(SpAr
     for (int i = 0; i < DB; i++)
 #pragma unroll
         for (int r = 0; r < 16; r++) O[i][r] = 0.f;
-    float bsum[G], lsum = 0.f, m = -1e30f;
+    float bsum[G], lsum = 0.f, m = -__builtin_inff();      // m: -inf until the row sees a key
 #pragma unroll
     for (int g = 0; g < G; g++) bsum[g] = 0.f;
 
@@ -341,7 +341,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void sdpa_prefill_kernel(SpAr
             if (__any(mx > m + 8.0f)) {
                 // per row: what a row's neighbours score does not move its maximum
                 const float mn = mx > m + 8.0f ? mx : m;
-                const float f = __builtin_amdgcn_exp2f((m - mn) * SP_LOG2E);
+                const float f = mn == m ? 1.0f : __builtin_amdgcn_exp2f((m - mn) * SP_LOG2E);
                 m = mn;
                 lsum *= f;
 #pragma unroll
@@ -351,7 +351,16 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void sdpa_prefill_kernel(SpAr
 #pragma unroll
                     for (int r = 0; r < 16; r++) O[i][r] *= f;
             }
-            const float mb = m * SP_LOG2E;
+            // e^(S - m): one multiply-add per score while the rounding of m log2(e)
+            // is under 2^-16; rows that have seen no key and larger scores
+            // subtract m first
+            float mb = m * SP_LOG2E;
+            if (__any(!(__builtin_fabsf(m) <= 256.0f))) {
+                const float ms = m == -__builtin_inff() ? 0.0f : m;
+#pragma unroll
+                for (int r = 0; r < 16; r++) S[r] -= ms;
+                mb = 0.0f;
+            }
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 S[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(S[r], SP_LOG2E, -mb));
@@ -430,7 +439,7 @@ __global__ __launch_bounds__(256) void sdpa_merge(const float* __restrict__ po, 
     if (i >= rows * cpr) return;
     const int64_t row = i / cpr;
     const int c = (int)(i % cpr);
-    float m = -1e30f;
+    float m = -__builtin_inff();
     for (int s = 0; s < splits; s++) m = __builtin_fmaxf(m, pm[s * rows + row].x);
     f32x4 o = {0.f, 0.f, 0.f, 0.f};
     float l = 0.f;

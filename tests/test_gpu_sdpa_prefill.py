@@ -92,3 +92,30 @@ def test_a_row_does_not_depend_on_its_neighbours(dev):
     same[0, 1, 37] = False
     assert torch.equal(got[same], ref[same])
     assert not torch.equal(got[~same], ref[~same])
+
+
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("size,N,mask", [(1e30, 100, None), (1e36, 700, "causal"), (2.4e38, 100, None),
+                                         (2.4e38, 700, "causal")])
+def test_scores_of_any_finite_size(dev, size, sign, N, mask):
+    """Scores far past float32's exponential, up to bf16's largest numbers:
+    each row's softmax is 1 at its largest score, as the separate products
+    give it.  Codes of 0, so a score is the sum of the group biases times the
+    query; key N - 9 wins (positive) or loses least (negative) by a sixteenth,
+    rows that do not see it share their weight over all keys."""
+    L, D = 64, 128
+    rng = np.random.default_rng(12)
+    _, tV = _kv(rng, 1, 1, N, D, 8, dev)
+    kb = torch.full((1, 1, N, 2), 1.0, dtype=BF, device=dev)
+    kb[0, 0, N - 9] = 1.0625 if sign > 0 else 0.9375
+    tK = (torch.zeros(1, 1, N, 32, dtype=torch.int32, device=dev), torch.zeros(1, 1, N, 2, dtype=BF, device=dev), kb)
+    q = torch.full((1, 1, L, D), sign * size / D, dtype=BF, device=dev)
+    assert kvattn._prefill_strides(q, tK, tV, mask, 64, 8) is not None
+    got = kvattn.quantized_sdpa(q, tK, tV, 1.0, mask)
+    V = torch.from_numpy(O.dequantize(tV[0].view(torch.int32).cpu().numpy().view(np.uint32), to_numpy(tV[1]),
+                                      to_numpy(tV[2]), 64, 8)).reshape(N, D)
+    ref = torch.empty(L, D)
+    for l in range(L):
+        last = N if mask is None else N - L + l + 1
+        ref[l] = V[N - 9] if N - 9 < last else V[:last].mean(0)
+    assert_close(to_numpy(got)[0, 0], ref.numpy(), what=f"scores of {sign * size}")
