@@ -261,7 +261,9 @@ def _prefill_strides(q, K, V, mask, group: int, bits: int):
     if D not in (64, 128, 256) or q.dtype != torch.bfloat16 or not q.is_cuda:
         return None
     shape = tuple(K[0].shape[:-1])
-    if len(shape) != 3 or shape[0] != B or H // shape[1] * L < PREFILL_ROWS or shape[2] < (1 if mask is None else L):
+    if len(shape) != 3 or shape[0] != B or B == 0 or H // shape[1] * L < PREFILL_ROWS:
+        return None
+    if shape[2] < (1 if mask is None else L):
         return None
     st = []
     for w, s, b in (K, V):

@@ -119,3 +119,13 @@ def test_scores_of_any_finite_size(dev, size, sign, N, mask):
         last = N if mask is None else N - L + l + 1
         ref[l] = V[N - 9] if N - 9 < last else V[:last].mean(0)
     assert_close(to_numpy(got)[0, 0], ref.numpy(), what=f"scores of {sign * size}")
+
+
+@pytest.mark.parametrize("mask", [None, "causal"])
+def test_an_empty_batch_keeps_the_separate_products(dev, mask):
+    """One query head per KV head: an empty result, as it always was."""
+    rng = np.random.default_rng(13)
+    _, tK = _kv(rng, 1, 2, 96, 128, 8, dev)
+    none = tuple(t[:0] for t in tK)
+    q = torch.empty(0, 2, 64, 128, dtype=BF, device=dev)
+    assert kvattn.quantized_sdpa(q, none, none, 0.1, mask).shape == (0, 2, 64, 128)
