@@ -32,6 +32,10 @@
 // cores busy 25%); 120 queries over 882 keys 122 -> 26 us (one launch's host
 // work instead of three).  D = 256 holds one workgroup per CU: 512 queries x 16
 // heads over 2 KV heads, 4096 keys 229 -> 128, 300 over 2000 120 -> 107.
+// Chunks of 2048 queries over 4000 keys (few units, cut over all XCDs by
+// sp_place; a unit per XCD in brackets): 32 heads over 4, D = 128 1006 -> 229 (435),
+// 16 over 2, D = 256 765 -> 419 (1526). 
+#include "dispatch.hpp"
 #include "qgemv_dl.hpp"
 #include "../../include/knurlogic_amd.h"
 
@@ -102,12 +106,11 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void sdpa_prefill_kernel(SpAr
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, h = lane >> 5;
-    // workgroup -> (KV head and split, row tile): the row tiles of a head's
-    // split share an XCD, whose L2 then holds its K and V
-    const int units = a.BHk * a.splits;
-    const int id = (int)blockIdx.x, xcd = id & 7, kk = id >> 3;
-    const int unit = 8 * (kk / a.row_tiles) + xcd, tile = kk % a.row_tiles;
-    if (unit >= units) return;
+    // workgroup -> (KV head and split, row tile): neighbours share an XCD,
+    // whose L2 then holds their K and V
+    const SpPlace wg = sp_place((int)blockIdx.x, a.BHk * a.splits, a.row_tiles);
+    if (wg.unit < 0) return;
+    const int unit = wg.unit, tile = wg.tile;
     const int head = unit / a.splits, split = unit % a.splits;
     const int64_t bi = head / a.Hk, hi = head % a.Hk;
 
@@ -480,14 +483,14 @@ SpPlan sp_plan(int64_t BHk, int64_t rows, int64_t N, int64_t D) {
 
 template <int BITS, int D>
 int sp_go(const SpArgs& a, hipStream_t st) {
-    const int64_t wgs = 8 * (int64_t)a.row_tiles * ceil_div((int64_t)a.BHk * a.splits, 8);
+    const int64_t wgs = (int64_t)a.BHk * a.splits * a.row_tiles + SP_XCDS;
     if (wgs >= (1LL << 31)) {
         set_error("sdpa_prefill: grid of %lld workgroups", (long long)wgs);
         return EINVAL_ARG;
     }
     constexpr size_t lds = 2 * SpShape<BITS, D>::STAGE;
     allow_dynamic_lds_once((const void*)sdpa_prefill_kernel<BITS, D>);
-    sdpa_prefill_kernel<BITS, D><<<(unsigned)wgs, 256, lds, st>>>(a);
+    sdpa_prefill_kernel<BITS, D><<<SP_XCDS * sp_run(a.BHk * a.splits, a.row_tiles), 256, lds, st>>>(a);
     KMI_CHECK_LAUNCH("sdpa_prefill");
     return OK;
 }
