@@ -434,8 +434,60 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void sdpa_prefill_kernel(SpAr
     }
 }
 
-// out[row, 4 c ..] = sum_s e^(m_s - m) o_s / sum_s e^(m_s - m) l_s, splits in order
+// out[row] = sum_s w_s o_s / sum_s w_s l_s, w_s = e^(m_s - m): a workgroup per
+// row, its splits dealt to 256 / (D / 4) groups of threads (each sums its own in
+// order, the groups' sums are added in order), so few rows' loads are in
+// flight together: 128 rows of 50 splits, D = 256 25 us with a thread per 4
+// columns, 5 here; but 16384 rows of 4 splits, D = 128 7 and 17 us.
+constexpr int SP_MAX_SPLITS = 512;
+
+template <int D>
 __global__ __launch_bounds__(256) void sdpa_merge(const float* __restrict__ po, const float2* __restrict__ pm,
+                                                  int splits, int64_t rows, uint16_t* __restrict__ out) {
+    constexpr int CPR = D / 4, NG = 256 / CPR;
+    __shared__ float wgt[SP_MAX_SPLITS];
+    __shared__ f32x4 part[256];
+    const int tid = threadIdx.x, lane = tid & 63, c = tid % CPR, g = tid / CPR;
+    const int64_t row = blockIdx.x;
+    // every wave forms m and sum_s w_s l_s
+    float m = -__builtin_inff();
+    for (int s = lane; s < splits; s += 64) m = __builtin_fmaxf(m, pm[s * rows + row].x);
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) m = __builtin_fmaxf(m, __shfl_xor(m, d, 64));
+    float l = 0.f;
+    for (int s = lane; s < splits; s += 64) {
+        const float2 ml = pm[s * rows + row];
+        const float f = __builtin_amdgcn_exp2f((ml.x - m) * SP_LOG2E);
+        if (tid < 64) wgt[s] = f;
+        l = __builtin_fmaf(f, ml.y, l);
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) l += __shfl_xor(l, d, 64);
+    __syncthreads();
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int s = g; s < splits; s += NG) {
+        const f32x4 v = *(const f32x4*)(po + (s * rows + row) * D + 4 * c);
+        const float f = wgt[s];
+#pragma unroll
+        for (int j = 0; j < 4; j++) o[j] = __builtin_fmaf(f, v[j], o[j]);
+    }
+    part[tid] = o;
+    __syncthreads();
+    if (g > 0) return;
+#pragma unroll
+    for (int q = 1; q < NG; q++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) o[j] += part[q * CPR + c][j];
+    const float inv = 1.0f / l;
+    u32x2 v;
+    v.x = cvt_pk_bf16(o[0] * inv, o[1] * inv);
+    v.y = cvt_pk_bf16(o[2] * inv, o[3] * inv);
+    *(u32x2*)(out + row * D + 4 * c) = v;
+}
+
+// The same with a thread per 4 columns: many rows of few splits.
+__global__ __launch_bounds__(256) void sdpa_merge_flat(const float* __restrict__ po, const float2* __restrict__ pm,
                                                   int splits, int64_t rows, int D, uint16_t* __restrict__ out) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int cpr = D / 4;
@@ -446,6 +498,7 @@ __global__ __launch_bounds__(256) void sdpa_merge(const float* __restrict__ po, 
     for (int s = 0; s < splits; s++) m = __builtin_fmaxf(m, pm[s * rows + row].x);
     f32x4 o = {0.f, 0.f, 0.f, 0.f};
     float l = 0.f;
+#pragma unroll 4
     for (int s = 0; s < splits; s++) {
         const float2 ml = pm[s * rows + row];
         const float f = __builtin_amdgcn_exp2f((ml.x - m) * SP_LOG2E);
@@ -466,17 +519,38 @@ struct SpPlan {
     size_t ws;
 };
 
-// Key splits until the grid has two workgroups per CU (D = 256: one), each
-// split at least 256 keys.
+// Key splits.  Until the grid has two workgroups per CU (D = 256: one), each
+// split at least 256 keys; or, where that is a long chain on few CUs, the split
+// with the least of: a workgroup's tiles of 64 keys (2.0 us each at D = 64, 2.8
+// at 128, 6.5 at 256) in rounds of the CUs, and the merge (10 us of launch and
+// host time, its bytes there and back at 3 TB/s), if it is 15% less by that
+// count.  Device time of 256-key splits alone, with this, and of the separate
+// products: 64 rows x 500 keys, 16 heads over 2, D = 256 59, 18, 24 us; 8 heads
+// over 1, D = 128 26, 13, 21; 72 rows x 16000 keys, D = 256 68, 32, 46.
 SpPlan sp_plan(int64_t BHk, int64_t rows, int64_t N, int64_t D) {
     SpPlan p;
     p.row_tiles = (int)ceil_div(rows, SP_ROWS);
-    const int64_t wgs = BHk * p.row_tiles, want = D > 128 ? 256 : 512;
-    int64_t s = wgs < want ? want / wgs : 1;
-    if (s > N / 256) s = N / 256 > 0 ? N / 256 : 1;
-    const int64_t kps = ceil_div(ceil_div(N, s), SP_KT) * SP_KT;
-    p.keys_per_split = (int)kps;
-    p.splits = (int)ceil_div(N, kps);
+    const int64_t wgs = BHk * p.row_tiles, slots = D > 128 ? 256 : 512, tiles = ceil_div(N, SP_KT);
+    const double tile_us = D > 128 ? 6.5 : D > 64 ? 2.8 : 2.0, split_us = 0.05 + (double)(BHk * rows) * D * 8 / 3e6;
+    auto cost = [&](int64_t per) {
+        const int64_t s = ceil_div(tiles, per);
+        return (double)ceil_div(wgs * s, slots) * per * tile_us + (s > 1 ? 10 + s * split_us : 0);
+    };
+    int64_t s0 = wgs < slots ? slots / wgs : 1;
+    if (s0 > N / 256) s0 = N / 256 > 0 ? N / 256 : 1;
+    int64_t best = ceil_div(ceil_div(N, s0), SP_KT);
+    double best_us = cost(best) * 0.85;
+    for (int64_t t = best;; t = t > 4 ? t * 3 / 4 : t - 1) {
+        const int64_t s = ceil_div(tiles, t), even = ceil_div(tiles, s);
+        if (s > SP_MAX_SPLITS) break;
+        if (cost(even) < best_us) {
+            best_us = cost(even);
+            best = even;
+        }
+        if (t == 1) break;
+    }
+    p.keys_per_split = (int)(best * SP_KT);
+    p.splits = (int)ceil_div(tiles, best);
     p.ws = p.splits > 1 ? (size_t)p.splits * BHk * rows * (D * 4 + 8) : 0;
     return p;
 }
@@ -556,7 +630,11 @@ int kmi_sdpa_prefill(const void* q, int64_t B, int64_t H, int64_t L, int64_t D, 
     if (rc) return rc;
     if (p.splits > 1) {
         const int64_t n = (int64_t)a.BHk * rows;
-        sdpa_merge<<<(unsigned)ceil_div(n * (D / 4), 256), 256, 0, st>>>(a.po, a.pm, p.splits, n, (int)D, a.out);
+        if (n * (D / 4) >= 512 * 256)
+            sdpa_merge_flat<<<(unsigned)ceil_div(n * (D / 4), 256), 256, 0, st>>>(a.po, a.pm, p.splits, n, (int)D, a.out);
+        else if (D == 64) sdpa_merge<64><<<(unsigned)n, 256, 0, st>>>(a.po, a.pm, p.splits, n, a.out);
+        else if (D == 128) sdpa_merge<128><<<(unsigned)n, 256, 0, st>>>(a.po, a.pm, p.splits, n, a.out);
+        else sdpa_merge<256><<<(unsigned)n, 256, 0, st>>>(a.po, a.pm, p.splits, n, a.out);
         KMI_CHECK_LAUNCH("sdpa_merge");
     }
     return OK;

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import oracle as O
-from knurlogic_amd import kvattn
+from knurlogic_amd import _abi, kvattn
 from tests.util import assert_close, bf16_normal, to_numpy, to_torch, u32_to_torch
 
 pytestmark = pytest.mark.gpu
@@ -129,3 +129,16 @@ def test_an_empty_batch_keeps_the_separate_products(dev, mask):
     none = tuple(t[:0] for t in tK)
     q = torch.empty(0, 2, 64, 128, dtype=BF, device=dev)
     assert kvattn.quantized_sdpa(q, none, none, 0.1, mask).shape == (0, 2, 64, 128)
+
+
+@pytest.mark.parametrize("B,H,Hk,L,N,D,bits,mask", [
+    (1, 2, 1, 32, 500, 256, 8, "causal"),      # a tile per split
+    (1, 2, 1, 40, 450, 128, 4, "causal"),
+    (1, 4, 2, 32, 700, 64, 8, None),
+    (1, 2, 1, 36, 8200, 128, 8, "causal"),     # tens of splits
+    (1, 8, 1, 1024, 600, 64, 8, None),         # enough rows for the merge by columns
+])
+def test_split_keys_match_the_oracle(dev, B, H, Hk, L, N, D, bits, mask):
+    """Key splits down to one tile and both merges."""
+    assert _abi.load().kmi_sdpa_prefill_workspace_bytes(B, H, Hk, L, N, D) > 0
+    test_matches_the_oracle(dev, B, H, Hk, L, N, D, bits, mask)
