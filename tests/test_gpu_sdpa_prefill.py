@@ -142,3 +142,36 @@ def test_split_keys_match_the_oracle(dev, B, H, Hk, L, N, D, bits, mask):
     """Key splits down to one tile and both merges."""
     assert _abi.load().kmi_sdpa_prefill_workspace_bytes(B, H, Hk, L, N, D) > 0
     test_matches_the_oracle(dev, B, H, Hk, L, N, D, bits, mask)
+
+
+@pytest.mark.parametrize("B,H,Hk,L,N,D,bits", [
+    (1, 2, 1, 600, 600, 128, 8),               # L = N: rows that see nothing of a later split, whole tiles among them
+    (1, 2, 2, 300, 900, 256, 8),
+    (1, 1, 1, 513, 520, 64, 4),
+])
+def test_key_splits_that_rows_do_not_see(dev, B, H, Hk, L, N, D, bits):
+    assert _abi.load().kmi_sdpa_prefill_workspace_bytes(B, H, Hk, L, N, D) > 0
+    test_matches_the_oracle(dev, B, H, Hk, L, N, D, bits, "causal")
+
+
+@pytest.mark.parametrize("step", [2.5, 9.0, 40.0])
+@pytest.mark.parametrize("D,N,mask", [(64, 130, None), (128, 700, "causal"), (256, 330, "causal"), (128, 16384, None)])
+def test_scores_that_climb_from_tile_to_tile(dev, step, D, N, mask):
+    """Scores that rise by `step` per tile of 64 keys for half of the rows and
+    fall for the others: the running maximum moves every few tiles, every
+    tile, and by far, what was summed before it must shrink with it (also the
+    biases' part, V far from zero), and key splits meet with maxima far
+    apart."""
+    rng = np.random.default_rng(int(step) + D + N)
+    H, L = 2, 40
+    u = rng.choice([-1.0, 1.0], D)
+    along = (np.arange(N) / 64 - N / 128) * step / 8               # q . u / D is 8 or -8
+    k = O.bf16_round((along[:, None] * u + rng.standard_normal((N, D)) * 0.3).astype(np.float32))[None, None]
+    K = O.quantize(k, 64, 8)
+    tK = (u32_to_torch(K[0], dev), to_torch(K[1], dev, BF), to_torch(K[2], dev, BF))
+    V, tV = _kv(rng, 1, 1, N, D, 8, dev, 2.0)
+    sign = np.where(np.arange(H * L) % 2, 1.0, -1.0).reshape(1, H, L, 1)
+    q = O.bf16_round((8 * sign * u + rng.standard_normal((1, H, L, D))).astype(np.float32))
+    got = kvattn.quantized_sdpa(to_torch(q, dev, BF), tK, tV, 1.0 / D, mask)
+    ref = O.quantized_sdpa(q, K, V, 1.0 / D, mask)
+    assert_close(to_numpy(got), ref, what="climbing scores")
