@@ -318,6 +318,10 @@ int launch_moe_eg(const QgArgs& a, int gs, bool glu, int64_t tile_slots, hipStre
         set_error("moe_eg: expert tiles of 4-bit affine weights, groups of 64 or 128");
         return EINVAL_ARG;
     }
+    if (!moe_eg_aligned(a.x, a.w, a.s, a.b)) {
+        set_error("moe_eg: x and weights on 16 bytes, scales and biases on 4");
+        return EINVAL_ARG;
+    }
     if (a.xrows * a.K * 2 >= (1LL << 31) || a.erows * (a.K / 2) >= (1LL << 31) || a.rows * a.N * 2 >= (1LL << 31)) {
         set_error("moe_eg: x, y or an expert's weights past 2 GiB");
         return EINVAL_ARG;

@@ -119,8 +119,11 @@ static int switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, int k
     KMI_CHECK_ARG(E <= 4096, "switch_glu: %lld experts (at most 4096)", (long long)E);
     KMI_CHECK_ARG(T * H * 2 < (1LL << 31) && T * k * (H > I ? H : I) * 2 < (1LL << 31),
                   "switch_glu: activations past 2 GiB");
-    const GluPlan p = plan_glu(T, H, I, k, E, moe_gemm_supported(H, I, bits, group_size, mx),
-                               moe_eg_supported(H, I, bits, group_size, mx));
+    // operands off moe_eg's alignment stay on moe_gemm (whose tiles are smaller
+    // than the skinny kernels' index space, so the queried workspace holds)
+    const bool eg_ok = moe_eg_supported(H, I, bits, group_size, mx) &&
+                       moe_eg_aligned(x, w_gu, s_gu, b_gu) && moe_eg_aligned(workspace, w_down, s_down, b_down);
+    const GluPlan p = plan_glu(T, H, I, k, E, moe_gemm_supported(H, I, bits, group_size, mx), eg_ok);
     KMI_CHECK_ARG(!mx || group_size == 32, "switch_glu (mx): group %d (32)", group_size);
     if (!workspace || workspace_bytes < p.total) {
         set_error("switch_glu: workspace of %zu bytes needed, %zu given", p.total, workspace_bytes);

@@ -84,6 +84,11 @@ int launch_moe_gemm(const QgArgs& a, int bits, int gs, bool glu, int tile_rows, 
 // The same over 4-bit weights (group 64 or 128, K % 64 == 0) in tiles of up to
 // moe_eg_tile_rows() rows whose cost follows their rows (moe_eg.hip).
 bool moe_eg_supported(int64_t H, int64_t I, int bits, int gs, int mx);
+// x and w on 16 bytes, s and b on 4: their 16-byte direct-to-LDS loads may not
+// start between words
+inline bool moe_eg_aligned(const void* x, const void* w, const void* s, const void* b) {
+    return (((uintptr_t)x | (uintptr_t)w) & 15u) == 0 && (((uintptr_t)s | (uintptr_t)b) & 3u) == 0;
+}
 int moe_eg_tile_rows();
 int launch_moe_eg(const QgArgs& a, int gs, bool glu, int64_t tile_slots, hipStream_t st);
 

@@ -143,3 +143,39 @@ def test_expert_tiles_at_their_edges(dev, h, i_, group):
     fns = [lambda xs, ex, m=m: O.quantized_matmul(xs, m[0][ex], m[1][ex], m[2][ex], True, group, 4, "bfloat16")
            for m in mats]
     assert_close(y[~bad], O.switch_glu(x[~bad], inds[~bad, None], *fns)[:, 0], what="expert tiles")
+
+
+@pytest.mark.parametrize("what", ["none", "x", "s_gu", "b_gu", "s_down", "b_down"])
+def test_expert_operands_at_any_element_offset(dev, what):
+    """64 experts of about 70 rows (moe_eg's sizes): operands that are views
+    off the alignment its loads need -- a scale or bias tensor at an odd
+    element, x at a 4-byte offset -- give the same result."""
+    from knurlogic_amd import ops
+    rng = np.random.default_rng(9400)
+    e, h, i_, k, T = 64, 320, 768, 4, 1120
+    t = {}
+    for name, N, Kd in (("gu", 2 * i_, h), ("down", h, i_)):
+        wq = np.frombuffer(rng.bytes(e * N * Kd // 2), np.uint32).reshape(e, N, Kd // 8)
+        sc = O.bf16_round(rng.uniform(0.004, 0.008, (e, N, Kd // 64)).astype(np.float32))
+        bi = O.bf16_round((-7.5 * sc + rng.normal(0, 0.002, sc.shape)).astype(np.float32))
+        t.update({f"w_{name}": u32_to_torch(wq, dev), f"s_{name}": to_torch(sc, dev, BF), f"b_{name}": to_torch(bi, dev, BF)})
+        if name == "gu":
+            gu = (wq, sc, bi)
+        else:
+            down = (wq, sc, bi)
+    x = bf16_normal(rng, (T, h))
+    t["x"] = to_torch(x, dev, BF)
+    if what != "none":
+        off = 2 if what == "x" else 1
+        flat = torch.empty(t[what].numel() + off, dtype=BF, device=dev)
+        view = flat[off:].view(t[what].shape)
+        view.copy_(t[what])
+        t[what] = view
+    inds = np.argsort(rng.random((T, e)), axis=1)[:, :k].astype(np.int32)
+    got = to_numpy(ops.switch_glu(t["x"], torch.from_numpy(inds).to(dev), t["w_gu"], t["s_gu"], t["b_gu"], t["w_down"],
+                                  t["s_down"], t["b_down"]))
+    part = lambda m, lo, hi: (lambda xs, ex: O.quantized_matmul(xs, m[0][ex, lo:hi], m[1][ex, lo:hi], m[2][ex, lo:hi],
+                                                                True, 64, 4, "bfloat16"))
+    s = _sample(rng, T)
+    ref = O.switch_glu(x[s], inds[s], part(gu, 0, i_), part(gu, i_, 2 * i_), part(down, 0, h))
+    assert_close(got[s], ref, what=f"{what} off its alignment")
