@@ -173,7 +173,9 @@ size_t kmi_qmm_mx_workspace_bytes(int64_t M, int64_t K, int64_t N, int mode);
  * first call with that device current).  Shapes whose partials need more
  * (kmi_qmm_workspace_bytes > KMI_QMM_SCRATCH_BYTES) are refused with -1.
  * The caller still allocates x and y.  All calls on one GPU share its
- * array: calls that overlap on one GPU (two streams or threads) race.
+ * array: calls that overlap on one GPU (two streams or threads) race, except
+ * at 65..128 rows, where K is not split (as kmi_qmm without a workspace) and
+ * the array is not touched.
  */
 #define KMI_QMM_SCRATCH_BYTES (32u << 20)
 size_t kmi_qmm_noalloc_scratch_bytes(void);

@@ -11,7 +11,10 @@
 // current) and passes that pointer to the kernels, never the name.
 //
 // Every call on a GPU shares that GPU's array: calls that overlap on one GPU
-// (two streams, two threads) race on it.  The kernels write every partial
+// (two streams, two threads) race on it -- but for 65..128 rows, which run
+// unsplit and leave it alone, as they did before the GEMM split K at these rows
+// (128 rows x [4096, 14336], 4-bit: 65 us unsplit, 36 with a workspace; 65 rows x
+// [14336, 4096] 213 and 33).  The kernels write every partial
 // they later read (split s writes all of its [M, N] slice before the
 // in-order reduce reads it), so nothing in the array has to start at zero
 // and the previous call's contents are never read.
@@ -64,7 +67,8 @@ size_t kmi_qmm_noalloc_scratch_bytes(void) { return KMI_QMM_SCRATCH_BYTES; }
 int kmi_qmm_noalloc(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w, const void* scales,
                     const void* biases, int dtype, int group_size, int bits, void* y, void* stream) {
     clear_error();
-    const size_t need = kmi_qmm_workspace_bytes(M, K, N, group_size, bits);
+    const bool unsplit = M > 64 && M <= 128;
+    const size_t need = unsplit ? 0 : kmi_qmm_workspace_bytes(M, K, N, group_size, bits);
     if (need > KMI_QMM_SCRATCH_BYTES) {
         set_error("quantized_matmul (no-alloc): M=%lld K=%lld N=%lld needs %zu bytes of split-K partials, "
                   "more than the %zu-byte scratch array; use kmi_qmm with a workspace",

@@ -96,3 +96,21 @@ def test_noalloc_matches_qmm_on_two_calls_in_a_row(dev):
     # 3) and one that needs no partials at all (single-row GEMV)
     need3, y3, z3 = _both(dev, 1, 4096, 4096, 4, 3)
     assert need3 == 0 and torch.equal(y3, z3)
+
+
+@pytest.mark.parametrize("M,K,N,bits", [(65, 4096, 4096, 4), (100, 14336, 1000, 8), (128, 4096, 14336, 4)])
+def test_noalloc_leaves_the_scratch_alone_from_65_to_128_rows(dev, M, K, N, bits):
+    """There the product is the unsplit one, bit for bit (kmi_qmm without a
+    workspace), although a workspace would split K: nothing is shared between
+    calls."""
+    torch.cuda.set_device(dev)
+    L = _abi.load()
+    need, y_ws, y_na = _both(dev, M, K, N, bits, M)
+    assert need > 0
+    x, w, s, b = _operands(dev, M, K, N, bits, M)
+    st = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    ref = torch.empty(M, N, dtype=BF, device=dev)
+    _abi.check(L.kmi_qmm(_ptr(x), M, K, N, _ptr(w), _ptr(s), _ptr(b), 0, 64, bits, _ptr(ref), None, 0, st), "qmm")
+    torch.cuda.synchronize()
+    assert torch.equal(y_na, ref)
+    assert not torch.equal(y_ws, ref)          # split sums round differently somewhere
