@@ -152,8 +152,8 @@ size_t kmi_qmm_workspace_bytes(int64_t M, int64_t K, int64_t N, int group_size, 
  * biases; fp32 accumulation, y rounded once to bf16 (x and y bf16).  Up to
  * 64 rows with K a multiple of 64 run kmi_qmm's decode kernels (M = 1: the
  * streaming GEMV; 2..16 rows with K a multiple of 256: the direct-to-LDS
- * MFMA kernel; else the MFMA GEMV), more rows kmi_qmm's MFMA GEMM (x 16-byte
- * aligned), anything else kmi_qmm_batched.  Each
+ * MFMA kernel; else the MFMA GEMV), more rows kmi_qmm's MFMA GEMM,
+ * anything else kmi_qmm_batched; past 64 rows x and w are 16-byte aligned.  Each
  * output row depends only on its own input row.  `workspace`
  * (kmi_qmm_mx_workspace_bytes) holds split-K partials; it may be NULL when
  * that size is 0.

@@ -415,7 +415,9 @@ int kmi_qmm_mx(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w
     KMI_CHECK_ARG(M >= 0 && K > 0 && K % 32 == 0 && N > 0,
                   "quantized_matmul: M=%lld K=%lld N=%lld (K a multiple of 32)", (long long)M, (long long)K,
                   (long long)N);
-    if (dtype == BF16 && x && w && scales && y && ((uintptr_t)x & 15u) == 0 && mx_gemm_shape(M, K, N, bits))
+    // (x or w off 16 bytes: the batched kernel's refusal)
+    if (dtype == BF16 && x && w && scales && y && (((uintptr_t)x | (uintptr_t)w) & 15u) == 0 &&
+        mx_gemm_shape(M, K, N, bits))
         return qmm_gemm_mx(x, M, K, N, w, scales, bits, y, workspace, workspace_bytes, (hipStream_t)stream);
     if (!mx_decode_shape(M, K)) {
         const int64_t xs[1] = {K}, ws[1] = {K * bits / 32}, ss[1] = {K / 32};

@@ -83,3 +83,19 @@ def test_up_to_128_rows_without_scratch(dev, mode):
         ref = ops.quantized_matmul(x, w, ts, None, True, 32, 4, "mxfp4")
     assert rc == 0
     assert_close(to_numpy(y), to_numpy(ref), what="no scratch")
+
+
+@pytest.mark.parametrize("which", ["x", "w"])
+def test_microscaled_rows_past_64_refuse_operands_off_16_bytes(dev, which):
+    """kmi_qmm_mx's C contract past 64 rows (the Python wrapper copies x)."""
+    from knurlogic_amd import _abi
+    lib = _abi.load()
+    M, N, K = 100, 300, 2048
+    x = torch.zeros(M * K + 8, dtype=BF, device=dev)
+    w = torch.zeros(N * K // 8 + 8, dtype=torch.int32, device=dev)
+    s = torch.full((N, K // 32), 120, dtype=torch.uint8, device=dev)
+    y = torch.zeros(M, N, dtype=BF, device=dev)
+    ws = torch.empty(lib.kmi_qmm_mx_workspace_bytes(M, K, N, 1), dtype=torch.uint8, device=dev)
+    rc = lib.kmi_qmm_mx(x.data_ptr() + (4 if which == "x" else 0), M, K, N, w.data_ptr() + (4 if which == "w" else 0),
+                        s.data_ptr(), 0, 1, y.data_ptr(), ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+    assert rc == -1 and b"16-byte aligned" in lib.kmi_last_error()
