@@ -153,7 +153,8 @@ size_t kmi_qmm_workspace_bytes(int64_t M, int64_t K, int64_t N, int group_size, 
  * 64 rows with K a multiple of 64 run kmi_qmm's decode kernels (M = 1: the
  * streaming GEMV; 2..16 rows with K a multiple of 256: the direct-to-LDS
  * MFMA kernel; else the MFMA GEMV), more rows kmi_qmm's MFMA GEMM,
- * anything else kmi_qmm_batched; past 64 rows x and w are 16-byte aligned.  Each
+ * anything else (and past 64 rows few outputs) kmi_qmm_batched; past 64 rows x
+ * and w are 16-byte aligned.  Each
  * output row depends only on its own input row.  `workspace`
  * (kmi_qmm_mx_workspace_bytes) holds split-K partials; it may be NULL when
  * that size is 0.

@@ -10,6 +10,7 @@
 // by sort_rows_by_expert, so each routed expert's weights are read once per
 // tile.
 #include "qmv_common.hpp"
+#include "dispatch.hpp"
 #include "qgemv.hpp"
 #include "../../include/knurlogic_amd.h"
 
@@ -392,7 +393,8 @@ int kmi_qmm(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w,
 
 // Microscaled dense: the decode kernels of kmi_qmm up to 64 rows and its GEMM
 // beyond, with the E2M1 / E4M3 decode and byte scales; K not a multiple of
-// 64, or a call past the GEMM's 2 GiB views, takes the batched kernel (nd = 0).
+// 64, a call past the GEMM's 2 GiB views, or one of few outputs
+// (mx_batched_wanted), takes the batched kernel (nd = 0).
 static bool mx_decode_shape(int64_t M, int64_t K) { return M <= SKINNY_MAX_M && K % 64 == 0; }
 static bool mx_gemm_shape(int64_t M, int64_t K, int64_t N, int bits) {
     return M > SKINNY_MAX_M && qmm_gemm_mx_fits(M, K, N, bits);
@@ -401,7 +403,7 @@ static bool mx_gemm_shape(int64_t M, int64_t K, int64_t N, int bits) {
 size_t kmi_qmm_mx_workspace_bytes(int64_t M, int64_t K, int64_t N, int mode) {
     if (M <= 0 || K <= 0 || N <= 0 || (mode != 1 && mode != 2)) return 0;
     const int bits = mode == 1 ? 4 : 8;
-    if (mx_gemm_shape(M, K, N, bits)) return qmm_gemm_workspace(M, K, N, bits);
+    if (mx_gemm_shape(M, K, N, bits) && !mx_batched_wanted(M, N, K)) return qmm_gemm_workspace(M, K, N, bits);
     if (!mx_decode_shape(M, K)) return kmi_qmm_batched_workspace_bytes(0, nullptr, M, K, N);
     if (choose_kind(M, K, bits) != QmvKind::SKINNY) return 0;
     return skinny_partial_bytes(dense_skinny_plan(M, K, N, bits, 32), M, N);
@@ -415,9 +417,12 @@ int kmi_qmm_mx(const void* x, int64_t M, int64_t K, int64_t N, const uint32_t* w
     KMI_CHECK_ARG(M >= 0 && K > 0 && K % 32 == 0 && N > 0,
                   "quantized_matmul: M=%lld K=%lld N=%lld (K a multiple of 32)", (long long)M, (long long)K,
                   (long long)N);
-    // (x or w off 16 bytes: the batched kernel's refusal)
+    // (x or w off 16 bytes: the batched kernel's refusal; without scratch for
+    // that kernel few outputs run on the GEMM, unsplit)
     if (dtype == BF16 && x && w && scales && y && (((uintptr_t)x | (uintptr_t)w) & 15u) == 0 &&
-        mx_gemm_shape(M, K, N, bits))
+        mx_gemm_shape(M, K, N, bits) &&
+        !(mx_batched_wanted(M, N, K) &&
+          (workspace ? workspace_bytes : 0) >= kmi_qmm_batched_workspace_bytes(0, nullptr, M, K, N)))
         return qmm_gemm_mx(x, M, K, N, w, scales, bits, y, workspace, workspace_bytes, (hipStream_t)stream);
     if (!mx_decode_shape(M, K)) {
         const int64_t xs[1] = {K}, ws[1] = {K * bits / 32}, ss[1] = {K / 32};

@@ -99,3 +99,23 @@ def test_microscaled_rows_past_64_refuse_operands_off_16_bytes(dev, which):
     rc = lib.kmi_qmm_mx(x.data_ptr() + (4 if which == "x" else 0), M, K, N, w.data_ptr() + (4 if which == "w" else 0),
                         s.data_ptr(), 0, 1, y.data_ptr(), ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
     assert rc == -1 and b"16-byte aligned" in lib.kmi_last_error()
+
+
+@pytest.mark.parametrize("mode", ["mxfp4", "mxfp8"])
+def test_few_microscaled_outputs_run_on_the_batched_kernel(dev, mode):
+    rng = np.random.default_rng(6)
+    M, N, K, bits = 100, 300, 2048, 4 if mode == "mxfp4" else 8
+    w = u32_to_torch(rng.integers(0, 100, (N, K * bits // 8), dtype=np.uint8).view(np.uint32), dev)
+    s = torch.from_numpy(rng.integers(115, 124, (N, K // 32), dtype=np.uint8)).to(dev)
+    x = to_torch(bf16_normal(rng, (M, K)), dev, BF)
+    assert torch.equal(ops.quantized_matmul(x, w, s, None, True, 32, bits, mode),
+                       ops.qmm_batched(x, w, s, None, True, 32, bits, mode=mode))
+
+
+@pytest.mark.parametrize("mode", ["mxfp4", "mxfp8"])
+@pytest.mark.parametrize("M,N,K", [(100, 2100, 2048), (300, 700, 1024), (129, 1100, 4096)])
+def test_microscaled_rows_with_k_splits(dev, M, N, K, mode):
+    """Outputs enough for the GEMM, few enough that it splits K."""
+    from knurlogic_amd import _abi
+    assert _abi.load().kmi_qmm_mx_workspace_bytes(M, K, N, 1 if mode == "mxfp4" else 2) > 0
+    test_microscaled_rows(dev, M, N, K, mode)
