@@ -480,6 +480,14 @@ int kmi_vq_glu(const void* x, int64_t T, int64_t H, int64_t I, int k, const int3
  */
 size_t kmi_vq_switch_glu_workspace_bytes(int64_t T, int64_t H, int64_t I, int k);
 /*
+ * Rows of the largest expert tile such a call runs in (one codebook for gate and
+ * up or two; the queried workspace, x and codes on 16 bytes): 1 a pair each, up to
+ * 16 expert tiles that gather every code per tile, more the grouped GEMM of
+ * prefill sizes.
+ */
+int kmi_vq_switch_glu_tile_rows(int64_t T, int64_t H, int64_t I, int k, int64_t E, int code_bytes, int kc,
+                                int shared_codebook);
+/*
  * VQSwitchLinear over the bit-packed on-disk code layout of the VQ
  * artifacts (src/knurlogic/engine/families/deepseek/heads/deepseek_v4.py:
  * 36-44,95-129; shipped as K = 2048 entries of dim 2-4 in 11-bit fields,
@@ -531,6 +539,9 @@ int kmi_vq_packed_glu(const void* x, int64_t X, int64_t H, int64_t I, const uint
  * decode.  workspace: kmi_vq_packed_switch_glu_workspace_bytes.
  */
 size_t kmi_vq_packed_switch_glu_workspace_bytes(int64_t T, int64_t H, int64_t I, int k);
+/* As kmi_vq_switch_glu_tile_rows (x on 16 bytes, scales on 4). */
+int kmi_vq_packed_switch_glu_tile_rows(int64_t T, int64_t H, int64_t I, int k, int64_t E, int pack_bits, int kc,
+                                       int dim, int group, int shared_codebook);
 int kmi_vq_packed_switch_glu(const void* x, int64_t T, int64_t H, int64_t I, int k, const int32_t* inds,
                              const void* scores, const uint32_t* codes_gate, const void* scales_gate,
                              const void* codebook_gate, const uint32_t* codes_up, const void* scales_up,

@@ -57,11 +57,13 @@ SIGNATURES = {
     "kmi_vq_gather_qmm": (I, [P, I64, I64, P, I, P, I, I, P, I, I64, I64, P, P, I64, I, P, P]),
     "kmi_vq_glu": (I, [P, I64, I64, I64, I, P, P, P, P, P, P, P, I, I, I, I, I64, I, P, P]),
     "kmi_vq_switch_glu_workspace_bytes": (SZ, [I64, I64, I64, I]),
+    "kmi_vq_switch_glu_tile_rows": (I, [I64, I64, I64, I, I64, I, I, I]),
     "kmi_vq_switch_glu": (I, [P, I64, I64, I64, I, P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I64, I,
                               P, P, SZ, P]),
     "kmi_vq_experts": (I, [P, P, I64, I64, I64, I, P, P, P, P, P, P, P, P, P, I, I, I, I, I64, I, P, P, P,
                            P, SZ, P]),
     "kmi_vq_packed_switch_glu_workspace_bytes": (SZ, [I64, I64, I64, I]),
+    "kmi_vq_packed_switch_glu_tile_rows": (I, [I64, I64, I64, I, I64, I, I, I, I, I]),
     "kmi_vq_packed_experts": (I, [P, P, I64, I64, I64, I, P, P, P, P, P, P, P, P, P, I, I, I, I, I64, I, P, P,
                                   P, P, SZ, P]),
     "kmi_vq_packed_switch_glu": (I, [P, I64, I64, I64, I, P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I64, I,

@@ -48,4 +48,57 @@ constexpr bool mx_batched_wanted(int64_t M, int64_t N, int64_t K) {
     return K >= 1024 && tiles <= 32 && tiles * (K / 64) <= 4000;
 }
 
+// ---- codebook experts: grouped GEMM or 16-row expert tiles (vq.hip, vq_packed.hip)
+// 32-row blocks of the largest tile the grouped GEMM takes, and its rows
+// (code_bytes 0: packed fields of vectors of dim)
+constexpr int vqg_max_blocks(int code_bytes, int dim) { return code_bytes ? 5 : dim == 2 ? 2 : 4; }
+constexpr int vqg_tile_rows(int code_bytes, int dim) { return 32 * vqg_max_blocks(code_bytes, dim); }
+
+// Whether P routed pairs over E experts, avg rows per routed expert, H -> I -> H,
+// run on the grouped GEMM (vq_gemm.hip) rather than on the 16-row expert tiles,
+// whose time grows with the rows while the GEMM's is nearly flat up to 32 rows
+// per expert.  The GEMM wants its gate/up grid to fill CUs (g: workgroups of a
+// largest tile and 256 output columns, one per CU) and rows enough per tile, the
+// fewer the more inputs share what a tile sets up; g, rows and H trade.  The
+// lines come from 2020 calls timed on both, 4 to 128 experts, 1024..3072 -> 256..1536,
+// 3 to 400 rows; none takes the kernel that was over 2% slower.  Nearest to them,
+// 16-row tiles and GEMM, us:
+//   one-byte codes: 128 experts 2048 -> 768 (g 384), 16 rows 112 and 103; 40 experts
+//     (g 120), 47 rows 88 and 78; 32 experts (g 96), 32 rows 63 and 63; 1024 -> 512: 60
+//     experts (g 120), 24 rows 47 and 48, 32 experts (g 64), 128 rows 74 and 85, 8 experts (g
+//     16) 37 and 77; 1536 -> 1024: 128 experts, 16 rows 98 and 103, 96 experts, 30 rows
+//     123 and 110.
+//   16-bit codes (a tile stages its codebook, 64 KB at 4096 x 8): 128 experts 2048 ->
+//     768, 3 rows 117 and 108; 48 experts 2048 -> 512 (g 96), 7 rows 69 and 52; 16 experts 2048
+//     -> 768 (g 48), 32 rows 75 and 62; 8 experts (g 24), 128 rows 93 and 108; 1024 -> 512:
+//     128 experts (g 256), 3 rows 44 and 49; 60 experts (g 120), 8 rows 41 and 43; 32 experts
+//     (g 64), 16 rows 42 and 42, 32 rows 51 and 49; 16 experts (g 32), 32 rows 44 and 47.
+//   packed vectors of 4 and 8 (11-bit x 4): 128 experts 2048 -> 768, 5 rows 185 and 160;
+//     32 experts (g 96), 12 rows 84 and 70; 16 experts 2048 -> 512 (g 32), 24 rows 59 and 72;
+//     1280 -> 512: 32 experts (g 64), 12 rows 50 and 56, 24 rows 63 and 60; 8 experts (g 16),
+//     48 rows 45 and 58.
+//   vectors of 2: 128 experts 2816 -> 704, 17 rows 388 and 363; 24 experts 1024 -> 512 (g
+//     48), 56 rows 67 and 75; 24 experts 2048 -> 512 (g 48), 54 rows 137 and 108.
+constexpr bool vqg_wanted(int code_bytes, int dim, int64_t P, int64_t E, int64_t avg, int64_t H, int64_t I) {
+    const int64_t blocks = vqg_max_blocks(code_bytes, dim), full = avg / (32 * blocks);
+    const int64_t rest = rule_ceil_div(avg - full * 32 * blocks, 32);
+    const int64_t g = (P < E ? P : E) * rule_ceil_div(I, 256) * (full ? full * blocks + rest : rest) /
+                      (full ? blocks : rest ? rest : 1);
+    const bool wide = H >= 2048;
+    if (code_bytes == 2) {
+        if (H >= 1536)
+            return (wide && g >= 384 && avg >= 3) || (g >= 128 && avg >= 6) || (g >= 96 && avg >= 7) ||
+                   (g >= 80 && avg >= 9) || (g >= 64 && avg >= 19) || (wide && g >= 48 && avg >= 32) ||
+                   (g >= 38 && avg >= 120);
+        return (g >= 128 && avg >= 10) || (g >= 80 && avg >= 24) || (g >= 64 && avg >= 38) || (g >= 48 && avg >= 140);
+    }
+    if (code_bytes == 1)
+        return P >= 1024 && ((g >= 128 && avg >= (H >= 2 * I ? 16 : 24)) || (g >= 96 && avg >= (wide ? 40 : 64)) ||
+                             (wide && g >= 72 && avg >= 200));
+    if (dim == 2) return P >= 1024 && avg >= 17 && (g >= 56 || (g >= 40 && (wide || avg >= 140)));
+    if (P < 384 || avg < (P >= 640 ? 5 : 12)) return false;
+    return g >= 128 || (g >= 96 && avg >= (wide ? 12 : 16)) || (g >= 80 && avg >= 18) || (g >= 64 && avg >= 24) ||
+           (g >= (wide ? 32 : 40) && avg >= 36) || (wide && g >= 27 && avg >= 140);
+}
+
 }  // namespace kmi

@@ -452,6 +452,28 @@ static bool vq_route_in_kernel(int64_t T, int64_t H, int k, int64_t E, int code_
            vq_mfma_supported(H, code_bytes, kc, two_cb);
 }
 
+// Tile rows of the 16-row path: LDS holds a tile's x rows, sized for the
+// largest tile, so few routed rows per expert take 4- or 8-row tiles (more
+// workgroups fit a CU); the sort cuts every expert's rows into tiles of at
+// most this.  One token: its k pairs are their own tiles (pair mode), no sort.
+static int vq_tile_rows(int64_t T, int k, int64_t E) {
+    const int64_t P = T * k, avg = ceil_div(P, E < P ? E : P);
+    const int rows = avg <= 2 ? 4 : avg <= 4 ? 8 : VQM_TILE_ROWS;
+    return T == 1 ? 1 : rows > P ? (int)P : rows;
+}
+
+// Prefill: rows grouped by expert in large tiles on the codebook GEMM (not where
+// the router's call would form its tiles, so both calls agree)
+static bool vq_grouped(int64_t T, int64_t H, int64_t I, int k, int64_t E, int code_bytes, int kc, int scale_group,
+                       bool two_cb) {
+    const int64_t P = T * k;
+    return T > 1 && scale_group == 0 && E <= 4096 && P < (1LL << 24) && vq_mfma_supported(H, code_bytes, kc, two_cb) &&
+           vq_mfma_supported(I, code_bytes, kc, false) && !pair_tiles_fit(P, E, vq_tile_rows(T, k, E)) &&
+           vqg_wanted(code_bytes, 8, P, E, ceil_div(P, E < P ? E : P), H, I) && T * H * 2 < (1LL << 31) &&
+           P * (H > I ? H : I) * 2 < (1LL << 31) && vqg_supported(code_bytes, 0, 8, 0, E, I, H, kc, two_cb) &&
+           vqg_supported(code_bytes, 0, 8, 0, E, H, I, kc, false);
+}
+
 static int vq_switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, int k, const int32_t* inds,
                               const void* scores, const void* codes_gate, const void* scales_gate,
                               const void* codebook_gate, const void* codes_up, const void* scales_up,
@@ -489,26 +511,14 @@ static int vq_switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, in
         return EINVAL_ARG;
     }
     uint16_t* y = scores ? (uint16_t*)((char*)workspace + vq_act_bytes(T, I, k)) : (uint16_t*)out;
-    // one token: its k pairs are their own tiles (pair mode), no sort
     const bool pair_mode = T == 1;
-    // Tile rows: LDS holds a tile's x rows, sized for the largest tile, so
-    // few routed rows per expert take 4- or 8-row tiles (more workgroups fit a
-    // CU); the sort cuts every expert's rows into tiles of at most this.
-    const int64_t avg = ceil_div(P, E < P ? E : P);
-    int tile_rows = avg <= 2 ? 4 : avg <= 4 ? 8 : VQM_TILE_ROWS;
-    if (tile_rows > P) tile_rows = (int)P;
-    if (pair_mode) tile_rows = 1;
+    const int tile_rows = vq_tile_rows(T, k, E);
     // inds from the router (every expert in range) and few pairs: the MFMA
     // kernels form their tiles themselves, no sort
     const bool formed = routed && !pair_mode && pair_tiles_fit(P, E, tile_rows);
-    // Prefill: rows grouped by expert in large tiles on the codebook GEMM
-    // (not where the router's call would form its tiles, so both calls agree)
-    const bool gemm = m_glu && m_down && !pair_tiles_fit(P, E, tile_rows) && !pair_mode &&
-                      vqg_wanted(code_bytes, 8, P, avg) && al16(x) &&
+    const bool gemm = m_glu && m_down && al16(x) &&
                       workspace_bytes >= kmi_vq_switch_glu_workspace_bytes(T, H, I, k) &&
-                      T * H * 2 < (1LL << 31) && P * (H > I ? H : I) * 2 < (1LL << 31) &&
-                      vqg_supported(code_bytes, 0, 8, 0, E, I, H, kc, two_cb) &&
-                      vqg_supported(code_bytes, 0, 8, 0, E, H, I, kc, false);
+                      vq_grouped(T, H, I, k, E, code_bytes, kc, scale_group, two_cb);
     SortedRows sr = {};
     void* index_ws = (char*)workspace + vq_act_bytes(T, I, k) + vq_y_bytes(T, H, k);
     if (gemm) {
@@ -622,6 +632,13 @@ static int vq_switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, in
 }
 
 extern "C" {
+
+int kmi_vq_switch_glu_tile_rows(int64_t T, int64_t H, int64_t I, int k, int64_t E, int code_bytes, int kc,
+                                int shared_codebook) {
+    if (T <= 0 || H <= 0 || I <= 0 || k <= 0 || E <= 0) return 0;
+    if (vq_grouped(T, H, I, k, E, code_bytes, kc, 0, !shared_codebook)) return vqg_tile_rows(code_bytes, 8);
+    return vq_tile_rows(T, k, E);
+}
 
 int kmi_vq_switch_glu(const void* x, int64_t T, int64_t H, int64_t I, int k, const int32_t* inds,
                       const void* scores, const void* codes_gate, const void* scales_gate,

@@ -683,6 +683,26 @@ static bool vps_route_fits(int64_t P, int64_t E, int k, int pack_bits, int dim, 
            vp_lds(H, kc, dim, two_cb, true) <= 160 * 1024;
 }
 
+// tiles sized to the rows an expert sees: the LDS holds a tile's x rows, so
+// small tiles fit more workgroups per CU (T = 16 of 128 experts, top-8, 2048 x
+// 4: 8-row tiles 146 us, 4-row 117 us)
+static int vps_tile_rows(int64_t P, int64_t E) {
+    const int64_t avg = ceil_div(P, E < P ? E : P);
+    const int rows = (int)(avg <= 2 ? 4 : avg <= 4 ? 8 : VPM_TILE);
+    return rows > P ? (int)P : rows;
+}
+
+// Prefill: large expert tiles on the codebook GEMM (not where the router's call
+// would form its tiles, so both calls agree)
+static bool vps_large_tiles(int64_t T, int64_t H, int64_t I, int k, int64_t E, int pack_bits, int kc, int dim, int group,
+                            bool two_cb) {
+    const int64_t P = T * k, Wg = (H / dim + 31) / 32 * pack_bits, Wd = (I / dim + 31) / 32 * pack_bits;
+    return vps_grouped(P, E, pack_bits, dim, group, H, I, kc, two_cb) && !pair_tiles_fit(P, E, vps_tile_rows(P, E)) &&
+           vqg_wanted(0, dim, P, E, ceil_div(P, E < P ? E : P), H, I) && I * Wg * 4 < (1LL << 31) &&
+           H * Wd * 4 < (1LL << 31) && vqg_supported(0, pack_bits, dim, group, E, I, H, kc, two_cb) &&
+           vqg_supported(0, pack_bits, dim, group, E, H, I, kc, false);
+}
+
 // The packed SwitchGLU.  With logits (per-pair path, E <= 256, k <= 8) the
 // gate/up kernel routes each pair's token and writes inds / scores, which
 // the down kernel and the combine read.
@@ -723,25 +743,15 @@ static int vps_switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, i
         return EINVAL_ARG;
     }
     if (grouped) {
-        const int64_t avg = ceil_div(P, E < P ? E : P);
-        // tiles sized to the rows an expert sees: the LDS holds a tile's x rows,
-        // so small tiles fit more workgroups per CU (T = 16 of 128 experts,
-        // top-8, 2048 x 4: 8-row tiles 146 us, 4-row 117 us)
-        int tile_rows = (int)(avg <= 2 ? 4 : avg <= 4 ? 8 : VPM_TILE);
-        if (tile_rows > P) tile_rows = (int)P;
+        const int tile_rows = vps_tile_rows(P, E);
         // inds from the router (every expert in range) and few pairs: the
         // kernels form their tiles themselves, no sort
         const bool formed = routed && pair_tiles_fit(P, E, tile_rows);
         SortedRows sr = {};
         int32_t* const list = (int32_t*)((char*)workspace + vps_act_bytes(P, I) + vps_y_bytes(P, H));
-        // Prefill: large expert tiles on the codebook GEMM (not where the
-        // router's call would form its tiles, so both calls agree)
-        if (!pair_tiles_fit(P, E, tile_rows) && vqg_wanted(0, dim, P, avg) && ((uintptr_t)x & 15u) == 0 &&
-            workspace_bytes >= kmi_vq_packed_switch_glu_workspace_bytes(T, H, I, k) &&
+        if (((uintptr_t)x & 15u) == 0 && workspace_bytes >= kmi_vq_packed_switch_glu_workspace_bytes(T, H, I, k) &&
             (((uintptr_t)scales_gate | (uintptr_t)scales_up | (uintptr_t)scales_down) & 3u) == 0 &&
-            I * Wg * 4 < (1LL << 31) && H * Wd * 4 < (1LL << 31) &&
-            vqg_supported(0, pack_bits, dim, group, E, I, H, kc, two_cb) &&
-            vqg_supported(0, pack_bits, dim, group, E, H, I, kc, false)) {
+            vps_large_tiles(T, H, I, k, E, pack_bits, kc, dim, group, two_cb)) {
             rc = launch_sort_rows(inds, P, 1, (int)E, vqg_tile_rows(0, dim), list, y, H, st, &sr);
             if (rc) return rc;
             uint16_t* x16 = (uint16_t*)((char*)list + sort_index_bytes(P, 4096, 1));
@@ -841,6 +851,13 @@ static int vps_switch_glu_impl(const void* x, int64_t T, int64_t H, int64_t I, i
 }
 
 extern "C" {
+
+int kmi_vq_packed_switch_glu_tile_rows(int64_t T, int64_t H, int64_t I, int k, int64_t E, int pack_bits, int kc, int dim,
+                                       int group, int shared_codebook) {
+    if (T <= 0 || H <= 0 || I <= 0 || k <= 0 || E <= 0 || (dim != 2 && dim != 4 && dim != 8)) return 0;
+    if (vps_large_tiles(T, H, I, k, E, pack_bits, kc, dim, group, !shared_codebook)) return vqg_tile_rows(0, dim);
+    return vps_grouped(T * k, E, pack_bits, dim, group, H, I, kc, !shared_codebook) ? vps_tile_rows(T * k, E) : 1;
+}
 
 int kmi_vq_packed_switch_glu(const void* x, int64_t T, int64_t H, int64_t I, int k, const int32_t* inds,
                              const void* scores, const uint32_t* codes_gate, const void* scales_gate,

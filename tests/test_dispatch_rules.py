@@ -16,6 +16,9 @@ int place(int id, int units, int tiles, int* tile) {
     *tile = p.tile;
     return p.unit;
 }
+int vqg(int cb, int dim, int64_t P, int64_t E, int64_t avg, int64_t H, int64_t I) {
+    return kmi::vqg_wanted(cb, dim, P, E, avg, H, I);
+}
 int mx_batched(int64_t M, int64_t N, int64_t K) { return kmi::mx_batched_wanted(M, N, K); }
 }
 """
@@ -29,6 +32,7 @@ def rules(tmp_path_factory):
                     "shim.so"], cwd=d, check=True)
     L = ctypes.CDLL(str(d / "shim.so"))
     L.mx_batched.argtypes = [ctypes.c_int64] * 3
+    L.vqg.argtypes = [ctypes.c_int] * 2 + [ctypes.c_int64] * 5
     return L
 
 
@@ -64,3 +68,67 @@ MX = [(65, 64, 2048, 12.9, 14.0), (65, 64, 14336, 16.1, 20.2), (128, 256, 4096, 
 @pytest.mark.parametrize("M,N,K,batched,gemm", MX)
 def test_microscaled_products_take_the_kernel_that_measured_faster(rules, M, N, K, batched, gemm):
     assert bool(rules.mx_batched(M, N, K)) == (batched < gemm)
+
+
+#: measured (us): 16-row expert tiles, the grouped GEMM -- (bytes per code or 0,
+#: vector, experts, routed pairs, H, I); the points nearest to even and some others
+VQ = [
+    (1, 8, 16, 1920, 1024, 256, 85.9, 90.2),
+    (1, 8, 128, 2048, 1536, 1024, 97.5, 102.8),
+    (1, 8, 16, 4800, 1024, 512, 84.4, 89.4),
+    (1, 8, 4, 1200, 1024, 512, 41.8, 79.4),
+    (1, 8, 8, 1024, 1024, 512, 36.6, 76.6),
+    (1, 8, 128, 2048, 2048, 768, 112.0, 103.2),
+    (1, 8, 48, 2640, 1024, 768, 71.8, 65.9),
+    (1, 8, 80, 1520, 1024, 512, 51.7, 47.1),
+    (1, 8, 96, 1536, 2048, 512, 73.2, 66.7),
+    (1, 8, 48, 14160, 2048, 768, 424.7, 238.8),
+    (1, 8, 128, 3584, 2048, 768, 167.4, 125.0),
+    (2, 8, 12, 324, 1024, 768, 45.4, 47.7),
+    (2, 8, 16, 512, 1024, 512, 44.4, 46.8),
+    (2, 8, 8, 264, 1024, 768, 46.9, 49.5),
+    (2, 8, 6, 412, 2048, 512, 41.8, 70.7),
+    (2, 8, 4, 512, 1024, 512, 45.3, 76.6),
+    (2, 8, 64, 640, 1024, 768, 49.9, 47.1),
+    (2, 8, 40, 360, 2048, 512, 56.6, 52.8),
+    (2, 8, 128, 384, 2048, 768, 116.7, 108.2),
+    (2, 8, 64, 448, 1536, 1024, 66.0, 60.5),
+    (2, 8, 32, 704, 2048, 1536, 126.5, 69.2),
+    (2, 8, 60, 7680, 2048, 768, 455.6, 136.1),
+    (0, 4, 12, 756, 2048, 512, 89.7, 95.6),
+    (0, 4, 8, 784, 1024, 768, 81.3, 87.1),
+    (0, 4, 16, 512, 1024, 768, 55.8, 60.3),
+    (0, 4, 4, 576, 1536, 512, 63.6, 95.1),
+    (0, 4, 4, 400, 1280, 512, 45.1, 85.2),
+    (0, 4, 20, 1160, 1536, 512, 94.5, 85.1),
+    (0, 4, 96, 864, 1024, 768, 93.7, 83.5),
+    (0, 4, 128, 1024, 1280, 512, 89.6, 78.9),
+    (0, 4, 16, 464, 1536, 1024, 83.7, 72.7),
+    (0, 4, 80, 4720, 2048, 768, 601.9, 154.1),
+    (0, 4, 48, 672, 2048, 512, 89.7, 69.9),
+    (0, 8, 4, 800, 3072, 512, 125.9, 133.8),
+    (0, 8, 12, 600, 1024, 256, 44.1, 47.3),
+    (0, 8, 16, 592, 1024, 256, 43.7, 47.2),
+    (0, 8, 4, 432, 2048, 512, 55.6, 101.1),
+    (0, 8, 4, 400, 1280, 512, 41.6, 81.4),
+    (0, 8, 32, 768, 1280, 512, 53.8, 50.6),
+    (0, 8, 32, 384, 2048, 768, 68.6, 63.3),
+    (0, 8, 128, 640, 1280, 512, 72.0, 63.5),
+    (0, 8, 16, 2080, 1536, 512, 109.8, 96.2),
+    (0, 8, 64, 7936, 1024, 512, 314.1, 107.7),
+    (0, 8, 128, 1920, 1536, 1024, 220.3, 117.5),
+    (0, 2, 24, 1344, 1024, 512, 67.1, 74.8),
+    (0, 2, 24, 1344, 1024, 512, 67.1, 74.8),
+    (0, 2, 40, 2720, 1024, 256, 80.3, 72.5),
+    (0, 2, 16, 2304, 1024, 256, 80.3, 72.4),
+    (0, 2, 8, 1520, 1024, 512, 85.0, 75.6),
+    (0, 2, 80, 1360, 2048, 512, 169.3, 149.6),
+    (0, 2, 128, 3072, 1280, 512, 180.9, 131.0),
+    (0, 2, 48, 5136, 1024, 256, 130.3, 74.3),
+]
+
+
+@pytest.mark.parametrize("cb,dim,E,P,H,I,tiles,gemm", VQ)
+def test_codebook_experts_take_the_kernel_that_measured_faster(rules, cb, dim, E, P, H, I, tiles, gemm):
+    avg = -(-P // min(E, P))
+    assert bool(rules.vqg(cb, dim, P, E, avg, H, I)) == (gemm < tiles)
