@@ -401,6 +401,13 @@ int kmi_switch_glu(const void* x, int64_t T, int64_t H, int64_t I, int k, const 
 
 size_t kmi_switch_glu_workspace_bytes(int64_t T, int64_t H, int64_t I, int k, int64_t E,
                                       int group_size, int bits);
+/*
+ * Rows of the largest expert tile such a call runs in (affine weights; x and
+ * weights on 16 bytes, scales and biases on 4): 1 token-major, up to 64 tiles of
+ * the skinny kernels, 128 or 256 the grouped GEMM, 160 the 4-bit tiles whose time
+ * follows their rows.
+ */
+int kmi_switch_glu_tile_rows(int64_t T, int64_t H, int64_t I, int k, int64_t E, int group_size, int bits);
 
 /*
  * kmi_switch_glu for experts stored in an OCP microscaled mode -- the

@@ -101,4 +101,37 @@ constexpr bool vqg_wanted(int code_bytes, int dim, int64_t P, int64_t E, int64_t
            (g >= (wide ? 32 : 40) && avg >= 36) || (wide && g >= 27 && avg >= 140);
 }
 
+// ---- 4-bit experts from 64 rows each: moe_eg's tiles or moe_gemm's -------------
+// Both run one workgroup per CU, so a projection takes rounds of the CUs.  A
+// moe_gemm round is a whole tile (128 rows x 256 weight rows, or 256 x 128 past 128
+// rows per expert) whatever it holds; moe_eg's workgroups take 512 weight rows and
+// their time follows their 32-row blocks, each 0.36 of a moe_gemm round.  Wins
+// where the experts' rows leave moe_gemm's tiles part empty or spill a few rows
+// into a second tile; loses where one round of moe_gemm holds them all.
+// moe_gemm and moe_eg, us: 128 experts 2048 -> 768, 64 rows 267 and 208, 128 rows
+// 412 and 277; 48 experts 1024 -> 768, 64 rows 97 and 73; 32 experts 2048 -> 1024, 80
+// rows 94 and 104, 128 rows 161 and 127; 16 experts 2048 -> 2048, 96 rows 106 and 124; 32
+// experts 1536 -> 512, 170 rows 85 and 99, 256 rows 132 and 103; 32 experts 1024 ->
+// 512, 166 rows 66 and 88, 317 rows 113 and 92.  Below half a grid (32 experts 1536
+// -> 512, 64 rows: 70 and 79) moe_gemm stays.
+constexpr int EG_MAX_BLOCKS = 5;             // row blocks of moe_eg's largest tile
+constexpr int64_t EG_MIN_GRID = 128;
+
+constexpr bool moe_eg_wanted(int64_t active, int64_t rows, int64_t H, int64_t I) {
+    constexpr int64_t TILE = 32 * EG_MAX_BLOCKS, CUS = 256;
+    if (active * rule_ceil_div(rows, TILE) * rule_ceil_div(I, 256) < EG_MIN_GRID) return false;
+    int64_t dev = 0;                         // routed rows spread by about their root
+    while ((dev + 1) * (dev + 1) <= rows) dev++;
+    const int64_t most = rows + dev;
+    const int64_t bm = rows <= 128 ? 128 : 256, tiles = active * rule_ceil_div(most, bm);
+    const int64_t gemm = rule_ceil_div(tiles * rule_ceil_div(I, 16384 / bm), CUS) * H +
+                         rule_ceil_div(tiles * rule_ceil_div(H, 32768 / bm), CUS) * I;
+    // row blocks of an expert, and of its largest tile
+    const int64_t full = most / TILE, rest = rule_ceil_div(most - full * TILE, 32);
+    const int64_t blocks = EG_MAX_BLOCKS * full + rest, largest = full ? EG_MAX_BLOCKS : rest;
+    const int64_t up = active * rule_ceil_div(I, 256) * blocks, down = active * rule_ceil_div(H, 512) * blocks;
+    const int64_t eg = (up > largest * CUS ? up : largest * CUS) * H + (down > largest * CUS ? down : largest * CUS) * I;
+    return 36 * eg < 100 * CUS * gemm;
+}
+
 }  // namespace kmi

@@ -21,6 +21,7 @@
 // moe_gemm, 180 here, down 131 -> 82 (what is left over the matrix cores' time:
 // 384 gate/up workgroups on 256 CUs, and 184 vector instructions of
 // dequantization per wave and stage beside 8 MFMAs per row block).
+#include "dispatch.hpp"
 #include "qgemv.hpp"
 
 namespace kmi {
@@ -45,7 +46,7 @@ __device__ __forceinline__ f32x16 eg_mfma(u32x4 a, u32x4 b, f32x16 c) {
 
 constexpr uint32_t EG_NONE = 0x80000000u;    // an offset past every view: reads 0
 constexpr int EG_BK = 64, EG_WAVES = 8;
-constexpr int EG_MAX_NB = 5;                 // row blocks of the largest tile
+constexpr int EG_MAX_NB = EG_MAX_BLOCKS;
 constexpr int EG_RIDS = 192;                 // tile rows staged (whole 64-row loads)
 constexpr int EG_CODES = 2048;               // a wave's codes per stage: 64 rows of 32 bytes
 

@@ -10,6 +10,7 @@
 // expert's weights are read once per call: gate|up with the SwiGLU
 // epilogue, then down, then the weighted combine.
 
+#include "dispatch.hpp"
 #include "moe_tok.hpp"
 #include "pair_tiles.hpp"
 #include "qgemv.hpp"
@@ -38,15 +39,10 @@ struct GluPlan {
 // Rows per active expert from which both projections run as a grouped GEMM
 // (prefill chunks: 64 rows fill four 16-row fragments of the skinny kernels)
 constexpr int64_t GEMM_MIN_ROWS = 64;
-// From the same row count 4-bit experts take moe_eg's tiles where its gate/up
-// grid (one workgroup per expert tile and 256 output columns, one per CU)
-// fills half of the CUs: 128 experts 2048 -> 768 -> 2048, 2048 tokens 400 us on
-// moe_gemm, 262 here, 1024 tokens 269 vs 225; 60 experts 1920 -> 704, 2048
-// tokens 218 vs 144; but 32 experts 1536 -> 512 at 64 rows each (64 workgroups)
-// 70 vs 79.  Below GEMM_MIN_ROWS the skinny kernels stay also where they are
-// slower (512 tokens 296 vs 193): they hold the weights exactly, this kernel
+// From the same row count 4-bit experts take moe_eg's tiles (moe_eg_wanted).
+// Below it the skinny kernels stay also where they are slower (512 tokens of 128
+// experts, 2048 -> 768 296 us, 193 on moe_eg): they hold the weights exactly, moe_eg
 // rounds them to bf16 as moe_gemm does.
-constexpr int64_t EG_MIN_GRID = 128;
 
 // rows per tile: the average routed pairs per active expert, in 16-row chunks
 // (gemm_ok, eg_ok: the grouped GEMMs take these weights)
@@ -62,8 +58,7 @@ static GluPlan plan_glu(int64_t T, int64_t H, int64_t I, int k, int64_t E, bool 
         // then stage their x rows once per workgroup (qgemv_xs) with two
         // workgroups per CU
         const int tm_skinny = rpt <= 2 ? 4 : qgemv_gather_tile_rows(rpt);
-        p.eg = eg_ok && rpt >= GEMM_MIN_ROWS &&
-               active * ceil_div(rpt, moe_eg_tile_rows()) * ceil_div(I, 256) >= EG_MIN_GRID;
+        p.eg = eg_ok && rpt >= GEMM_MIN_ROWS && moe_eg_wanted(active, rpt, H, I);
         p.gemm = !p.eg && gemm_ok && rpt >= GEMM_MIN_ROWS;
         p.tm = p.eg ? moe_eg_tile_rows() : p.gemm ? (rpt <= 128 ? 128 : 256) : tm_skinny;
         p.y = align256((size_t)P * H * 2);
@@ -86,6 +81,13 @@ size_t kmi_switch_glu_workspace_bytes(int64_t T, int64_t H, int64_t I, int k, in
     if (T <= 0 || H <= 0 || I <= 0 || k <= 0 || E <= 0) return 0;
     return plan_glu(T, H, I, k, E, moe_gemm_supported(H, I, bits, group_size, 0),
                     moe_eg_supported(H, I, bits, group_size, 0)).total;
+}
+
+int kmi_switch_glu_tile_rows(int64_t T, int64_t H, int64_t I, int k, int64_t E, int group_size, int bits) {
+    if (T <= 0 || H <= 0 || I <= 0 || k <= 0 || E <= 0) return 0;
+    const GluPlan p = plan_glu(T, H, I, k, E, moe_gemm_supported(H, I, bits, group_size, 0),
+                               moe_eg_supported(H, I, bits, group_size, 0));
+    return p.tok ? 1 : p.tm;
 }
 
 }  // extern "C"

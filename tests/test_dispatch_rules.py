@@ -19,6 +19,7 @@ int place(int id, int units, int tiles, int* tile) {
 int vqg(int cb, int dim, int64_t P, int64_t E, int64_t avg, int64_t H, int64_t I) {
     return kmi::vqg_wanted(cb, dim, P, E, avg, H, I);
 }
+int eg(int64_t active, int64_t rows, int64_t H, int64_t I) { return kmi::moe_eg_wanted(active, rows, H, I); }
 int mx_batched(int64_t M, int64_t N, int64_t K) { return kmi::mx_batched_wanted(M, N, K); }
 }
 """
@@ -32,6 +33,7 @@ def rules(tmp_path_factory):
                     "shim.so"], cwd=d, check=True)
     L = ctypes.CDLL(str(d / "shim.so"))
     L.mx_batched.argtypes = [ctypes.c_int64] * 3
+    L.eg.argtypes = [ctypes.c_int64] * 4
     L.vqg.argtypes = [ctypes.c_int] * 2 + [ctypes.c_int64] * 5
     return L
 
@@ -132,3 +134,39 @@ VQ = [
 def test_codebook_experts_take_the_kernel_that_measured_faster(rules, cb, dim, E, P, H, I, tiles, gemm):
     avg = -(-P // min(E, P))
     assert bool(rules.vqg(cb, dim, P, E, avg, H, I)) == (gemm < tiles)
+
+
+#: measured (us): moe_gemm, moe_eg -- (experts, rows each, H, I); the points nearest
+#: to even and some others
+EG = [
+    (16, 160, 2048, 2048, 143.3, 150.5),
+    (16, 170, 2048, 2048, 146.2, 157.9),
+    (16, 64, 2048, 2048, 101.9, 110.0),
+    (16, 80, 2048, 2048, 102.8, 111.6),
+    (16, 200, 2048, 2048, 152.3, 165.5),
+    (32, 96, 2048, 1024, 97.1, 106.8),
+    (32, 80, 2048, 1024, 94.4, 104.4),
+    (32, 200, 1536, 512, 88.4, 101.7),
+    (16, 96, 2048, 2048, 105.9, 123.9),
+    (32, 170, 1536, 512, 84.7, 99.2),
+    (32, 180, 2048, 512, 98.7, 118.1),
+    (32, 166, 1024, 512, 65.7, 88.1),
+    (64, 167, 1536, 512, 144.2, 132.8),
+    (40, 179, 2048, 512, 149.0, 137.1),
+    (8, 591, 1536, 1024, 126.5, 114.7),
+    (64, 74, 1536, 512, 89.2, 80.8),
+    (64, 194, 1536, 1024, 252.2, 227.8),
+    (40, 228, 2048, 1536, 323.3, 290.2),
+    (128, 200, 2048, 768, 500.8, 448.8),
+    (60, 160, 1920, 704, 226.5, 202.5),
+    (32, 330, 2048, 1024, 299.6, 255.0),
+    (32, 287, 1536, 1024, 220.5, 156.0),
+    (20, 396, 1024, 768, 114.4, 99.1),
+    (40, 514, 1024, 768, 260.6, 209.6),
+    (24, 466, 2048, 1536, 351.3, 299.7),
+]
+
+
+@pytest.mark.parametrize("E,rows,H,I,gemm,eg", EG)
+def test_4bit_experts_take_the_tiles_that_measured_faster(rules, E, rows, H, I, gemm, eg):
+    assert bool(rules.eg(E, rows, H, I)) == (eg < gemm)

@@ -179,3 +179,44 @@ def test_expert_operands_at_any_element_offset(dev, what):
     s = _sample(rng, T)
     ref = O.switch_glu(x[s], inds[s], part(gu, 0, i_), part(gu, i_, 2 * i_), part(down, 0, h))
     assert_close(got[s], ref, what=f"{what} off its alignment")
+
+
+@pytest.mark.parametrize("h,i_,group", [(320, 768, 64), (1024, 640, 128), (128, 704, 64)])
+def test_expert_tiles_at_their_edges_over_many_experts(dev, h, i_, group):
+    """As test_expert_tiles_at_their_edges over 64 experts, which the dispatch
+    puts on the tiles whose work follows their rows (the library's own query;
+    16 experts fit one round of the grouped GEMM)."""
+    from knurlogic_amd import _abi
+    rng = np.random.default_rng(9500 + h)
+    counts = [1, 31, 32, 33, 64, 65, 95, 127, 128, 129, 159, 160, 161, 330, 0] + [60] * 49
+    e, T = len(counts), sum(counts) + 2
+    i_ = i_ // group * group
+    assert _abi.load().kmi_switch_glu_tile_rows(T, h, i_, 1, e, group, 4) == 160
+    mats = []
+    for N, Kd in ((i_, h), (i_, h), (h, i_)):
+        wq = np.frombuffer(rng.bytes(e * N * Kd // 2), np.uint32).reshape(e, N, Kd // 8)
+        sc = O.bf16_round(rng.uniform(0.004, 0.008, (e, N, Kd // group)).astype(np.float32))
+        bi = O.bf16_round((-7.5 * sc + rng.normal(0, 0.002, sc.shape)).astype(np.float32))
+        mats.append((wq, sc, bi))
+    q = lambda m: nn.QuantizedSwitchLinear(u32_to_torch(m[0], dev), to_torch(m[1], dev, BF),
+                                           to_torch(m[2], dev, BF), None, group, 4)
+    glu = nn.SwitchGLU(*(q(m) for m in mats))
+    inds = np.concatenate([np.full(n, x) for x, n in enumerate(counts)] + [[e, -1]]).astype(np.int32)
+    rng.shuffle(inds)
+    x = bf16_normal(rng, (len(inds), h))
+    tx, ti = to_torch(x, dev, BF), torch.from_numpy(inds[:, None]).to(dev)
+    got = glu(tx, ti)
+    assert torch.equal(got, glu(tx, ti)), "a repeated call differs"
+    y, bad = to_numpy(got)[:, 0], (inds < 0) | (inds >= e)
+    assert (y[bad] == 0).all()
+    fns = [lambda xs, ex, m=m: O.quantized_matmul(xs, m[0][ex], m[1][ex], m[2][ex], True, group, 4, "bfloat16")
+           for m in mats]
+    assert_close(y[~bad], O.switch_glu(x[~bad], inds[~bad, None], *fns)[:, 0], what="expert tiles")
+
+
+def test_experts_that_fit_one_round_stay_on_the_grouped_gemm():
+    """(The library's host query; no GPU work.)"""
+    from knurlogic_amd import _abi
+    rows = lambda T, H, I, k, E: _abi.load().kmi_switch_glu_tile_rows(T, H, I, k, E, 64, 4)
+    assert rows(768, 2048, 2048, 2, 16) == 128 and rows(1328, 1024, 512, 4, 32) == 256
+    assert rows(2048, 2048, 768, 8, 128) == 160 and rows(1, 2048, 768, 8, 128) == 1
