@@ -438,7 +438,9 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void sdpa_prefill_kernel(SpAr
 // row, its splits dealt to 256 / (D / 4) groups of threads (each sums its own in
 // order, the groups' sums are added in order), so few rows' loads are in
 // flight together: 128 rows of 50 splits, D = 256 25 us with a thread per 4
-// columns, 5 here; but 16384 rows of 4 splits, D = 128 7 and 17 us.
+// columns, 5 here; but 16384 rows of 4 splits, D = 128 7 and 17 us.  (The whole
+// calls of 800 rows per KV head x 900 keys, D = 64, 8 heads, 4 splits: 28 us by rows,
+// 23 by columns; 256 rows x 1500 keys, D = 128, 1 head, 24 splits 14 and 19.)
 constexpr int SP_MAX_SPLITS = 512;
 
 template <int D>
@@ -630,7 +632,7 @@ int kmi_sdpa_prefill(const void* q, int64_t B, int64_t H, int64_t L, int64_t D, 
     if (rc) return rc;
     if (p.splits > 1) {
         const int64_t n = (int64_t)a.BHk * rows;
-        if (n * (D / 4) >= 512 * 256)
+        if (p.splits <= 6 || n * (D / 4) >= (p.splits <= 12 ? 256 : 512) * 256)
             sdpa_merge_flat<<<(unsigned)ceil_div(n * (D / 4), 256), 256, 0, st>>>(a.po, a.pm, p.splits, n, (int)D, a.out);
         else if (D == 64) sdpa_merge<64><<<(unsigned)n, 256, 0, st>>>(a.po, a.pm, p.splits, n, a.out);
         else if (D == 128) sdpa_merge<128><<<(unsigned)n, 256, 0, st>>>(a.po, a.pm, p.splits, n, a.out);
