@@ -17,10 +17,10 @@
 //     expert's scales and biases for the wave's rows are loaded once.
 //   - weights are bf16(s * q + b), one rounding, as moe_gemm's; the next MFMA
 //     step's are formed between this step's MFMAs, piece by piece.
-// Measured, 128 experts 2048 -> 768 -> 2048, top-8, 2048 tokens: gate/up 245 us on
-// moe_gemm, 180 here, down 131 -> 82 (what is left over the matrix cores' time:
-// 384 gate/up workgroups on 256 CUs, and 184 vector instructions of
-// dequantization per wave and stage beside 8 MFMAs per row block).
+// Measured, 128 experts 2048 -> 768 -> 2048, top-8, 2048 tokens: gate/up 256 us on
+// moe_gemm, 161 here, down 131 -> 87 (what is left over the matrix cores' time:
+// 384 gate/up workgroups on 256 CUs, and the dequantization's vector
+// instructions beside 8 MFMAs per row block).
 #include "dispatch.hpp"
 #include "qgemv.hpp"
 

@@ -161,15 +161,17 @@ struct QgemmArgs {
 // 128 x 256, waves 2 x 4, so no wave works on padding rows.
 // Measured (before: qmm_kernel up to 128 rows, its grid of N / 128 workgroups
 // with no K split; microscaled weights on the batched kernel, whose hi + lo
-// operands double the MFMAs): 4-bit 128 rows x [4096, 14336] 667 -> 36.5 us, 65
-// rows x [14336, 4096] 162 -> 33; 8-bit 100 rows x [4096, 4096] 158 -> 22;
-// mxfp4 1000 rows x [4096, 14336] 460 -> 127 (925 TFLOP/s), mxfp8 700 rows x
-// [5120, 2048] 77 -> 32.
+// operands double the MFMAs): 4-bit 128 rows x [4096, 14336] 663 -> 36 us, 65
+// rows x [14336, 4096] 162 -> 31; 8-bit 100 rows x [4096, 4096] 158 -> 22;
+// mxfp4 1000 rows x [4096, 14336] 459 -> 122 (960 TFLOP/s), mxfp8 700 rows x
+// [5120, 2048] 77 -> 33.
 //   - x and the dequantized weights are staged through LDS (two buffers),
 //     both loaded with 8 lanes per 128-byte row segment.  The weight tile is
 //     dequantized once per workgroup (fp32 s*q + b, one bf16 rounding: 16
-//     values per thread, 32 at 128 rows; microscaled codes as element * 2^e in
-//     fp32, which bf16 holds exactly).
+//     values per thread, 32 at 128 rows; microscaled codes as element * 2^(e - 127)
+//     in fp32, which bf16 holds exactly for E2M1 up to e = 252 and for E4M3
+//     from e = 3 to 246: beyond, the largest codes are infinite and E4M3's
+//     smallest fall below bf16's subnormals).
 //   - k order: in a k-tile, lane half h reads k in [32h, 32h + 32) and MFMA
 //     step s the 8 values 32h + 8s .. +8 of it, for x and w alike (the
 //     contraction is unchanged).

@@ -13,8 +13,8 @@
 // Every call on a GPU shares that GPU's array: calls that overlap on one GPU
 // (two streams, two threads) race on it -- but for 65..128 rows, which run
 // unsplit and leave it alone, as they did before the GEMM split K at these rows
-// (128 rows x [4096, 14336], 4-bit: 65 us unsplit, 36 with a workspace; 65 rows x
-// [14336, 4096] 213 and 33).  The kernels write every partial
+// (128 rows x [14336, 4096], 4-bit: 65 us unsplit, 36 with a workspace; 65 rows x
+// [4096, 14336] 213 and 33).  The kernels write every partial
 // they later read (split s writes all of its [M, N] slice before the
 // in-order reduce reads it), so nothing in the array has to start at zero
 // and the previous call's contents are never read.

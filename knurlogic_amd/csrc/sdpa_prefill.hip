@@ -27,14 +27,14 @@
 // Few rows leave CUs idle: the keys are then split, each split writing fp32
 // sums with its maximum, merged by sdpa_merge.
 // Measured, 512 queries x 32 heads over 4 KV heads, 8192 8-bit keys, D = 128: the
-// separate products 515 us (233 scores, 152 softmax, 257 P V), one pass 130
+// separate products 515 us (233 scores, 152 softmax, 257 P V), one pass 131
 // (vector instructions are issued 67% of the time, matrix
-// cores busy 25%); 120 queries over 882 keys 122 -> 26 us (one launch's host
+// cores busy 25%); 120 queries over 882 keys 118 -> 26 us (one launch's host
 // work instead of three).  D = 256 holds one workgroup per CU: 512 queries x 16
-// heads over 2 KV heads, 4096 keys 229 -> 128, 300 over 2000 120 -> 107.
+// heads over 2 KV heads, 4096 keys 229 -> 129, 300 over 2000 117 -> 62.
 // Chunks of 2048 queries over 4000 keys (few units, cut over all XCDs by
 // sp_place; a unit per XCD in brackets): 32 heads over 4, D = 128 1006 -> 229 (435),
-// 16 over 2, D = 256 765 -> 419 (1526). 
+// 16 over 2, D = 256 765 -> 419 (1526).
 #include "dispatch.hpp"
 #include "qgemv_dl.hpp"
 #include "../../include/knurlogic_amd.h"

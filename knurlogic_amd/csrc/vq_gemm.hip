@@ -28,10 +28,10 @@
 // are rounded as the other VQ kernels round (bf16 per projection, then the
 // SwiGLU's two roundings).
 // Measured, 128 experts 2048 -> 768 -> 2048, top-8: 4096 x 8 codebook, 2048
-// tokens 935 us on the 16-row tiles, 277 here (gate/up 158, down 78 us: the
-// matrix cores are busy 45% of a workgroup's time, and 384 gate/up workgroups
-// fill 256 CUs one and a half times); packed 2048 x 4, 512 tokens 544 -> 209
-// (gate/up 130: the address units, busy 63%, serve one weight row per lane).
+// tokens 934 us on the 16-row tiles, 257 here (gate/up 151, down 79 us: 384
+// gate/up workgroups fill 256 CUs one and a half times); packed 2048 x 4, 512
+// tokens 545 -> 179 (gate/up 109, down 53: the address units serve one weight
+// row per lane).
 #include "vq_gemm.hpp"
 
 #include <type_traits>
