@@ -15,7 +15,8 @@ Off the kernel, ``sdpa`` never computes attention in torch:
     caches, queries longer than the kernel takes, masks it does not take)
     -- go through ``quantized_sdpa``, mlx-lm's quantized attention
     (.../_mlx_vlm/models/base.py:260-302) over the packed triples: three
-    HIP launches, no dequantized copy of the cache;
+    HIP launches (a prompt chunk: one pass over the keys), no dequantized
+    copy of the cache;
   * dense K/V go to the model's own attention function, the one
     ``patch_model`` found and replaced (the reference likewise hands them
     to mlx-lm's base function).

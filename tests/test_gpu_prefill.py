@@ -116,10 +116,11 @@ def test_grouped_gemm_with_k_tiles_past_a_group(dev, bits):
 
 @pytest.mark.parametrize("h,i_,group", [(320, 1984, 64), (256, 2048, 128), (64, 2048, 64)])
 def test_expert_tiles_at_their_edges(dev, h, i_, group):
-    """4-bit experts on tiles whose work follows their rows (moe_eg.hip):
-    row counts around its 32-row blocks and its largest tile, an expert
-    without rows, columns that do not fill a column block, one and several
-    K stages, pairs whose expert is out of range."""
+    """4-bit experts of uneven rows, 16 of them (one round of the grouped
+    GEMM; over 64 experts below: the tiles whose work follows their rows,
+    moe_eg.hip): row counts around moe_eg's 32-row blocks and its largest
+    tile, an expert without rows, columns that do not fill a column block,
+    one and several K stages, pairs whose expert is out of range."""
     rng = np.random.default_rng(9300 + h)
     counts = [1, 31, 32, 33, 64, 65, 95, 127, 128, 129, 159, 160, 161, 330, 0, 40]
     e = len(counts)

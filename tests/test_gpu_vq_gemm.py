@@ -3,7 +3,8 @@ experts at prefill sizes) against the oracle's exact decode-then-matmul, at
 the edges of its 32-row blocks and largest tiles (one row, one short of a
 block, one past the largest tile), with columns that do not fill a column
 block, several K stages, pairs whose expert is out of range, and the layouts
-of the codes.  Bar: max rel err 1e-2, cosine 0.9999."""
+of the codes.  64 experts reach it; the same edges over 6 experts, which the
+dispatch leaves on the 16-row expert tiles, stand first.  Bar: max rel err 1e-2, cosine 0.9999."""
 import numpy as np
 import pytest
 import torch
