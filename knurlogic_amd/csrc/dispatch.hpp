@@ -9,30 +9,46 @@ namespace kmi {
 constexpr int64_t rule_ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // ---- the one-pass prompt attention's grid (sdpa_prefill.hip) -------------------
-// units (a KV head's key split) x row tiles, the units ordered by unit % 8 and
-// the whole cut into 8 runs of equal length, one per XCD (workgroup i runs on
-// XCD i % 8).  From 8 units on, a unit's tiles share an XCD's L2; at any
-// number no XCD is left with less.  (A whole unit per XCD left 4 of 8 idle at 4
-// units: sdpa_prefill.hip has both sides.  Neighbouring units, the key splits
-// of one head, on one XCD measured 3% slower at 16000 keys.)
-constexpr int SP_XCDS = 8;
+// units (a KV head's key split) x row tiles.  Unit u whole on XCD u % 8
+// (workgroup i runs on XCD i % 8), whose L2 then holds its K and V; where that
+// gives some XCD more workgroups per CU than an even share would, the units
+// ordered by u % 8 and the whole cut into 8 runs of equal length.  2048 queries over
+// 4000 keys, whole units and cut, us: 32 heads over 4 KV heads, D = 128 435 and
+// 229, 16 over 2, D = 256 1526 and 419; 300 x 3000, 16 over 2, D = 256 131 and 74.  Cut
+// without that need it is slower: 96 queries over 3387 keys, 32 over 4, D = 128 (44
+// units of 6 tiles: 36 workgroups on one XCD's 32 CUs, 33 if cut) 39 and 42.
+constexpr int SP_XCDS = 8, SP_XCD_CUS = 32;
 
 struct SpPlace {
     int unit, tile;         // unit -1: nothing to do
 };
 
-constexpr int sp_run(int units, int row_tiles) {
+// workgroups on the fullest XCD: whole units, and cut
+constexpr int sp_whole(int units, int row_tiles) { return (units + SP_XCDS - 1) / SP_XCDS * row_tiles; }
+constexpr int sp_cut(int units, int row_tiles) {
     return (int)rule_ceil_div((int64_t)units * row_tiles, SP_XCDS);
+}
+constexpr bool sp_is_cut(int units, int row_tiles) {
+    return (sp_whole(units, row_tiles) - 1) / SP_XCD_CUS > (sp_cut(units, row_tiles) - 1) / SP_XCD_CUS;
+}
+// the grid's workgroups per XCD
+constexpr int sp_run(int units, int row_tiles) {
+    return sp_is_cut(units, row_tiles) ? sp_cut(units, row_tiles) : sp_whole(units, row_tiles);
 }
 
 constexpr SpPlace sp_place(int id, int units, int row_tiles) {
-    const int run = sp_run(units, row_tiles), at = id % SP_XCDS * run + id / SP_XCDS;
-    if (id / SP_XCDS >= run || at >= units * row_tiles) return SpPlace{-1, 0};
+    const int run = sp_run(units, row_tiles), xcd = id % SP_XCDS, at = id / SP_XCDS;
+    if (at >= run) return SpPlace{-1, 0};
+    if (!sp_is_cut(units, row_tiles)) {
+        const int unit = SP_XCDS * (at / row_tiles) + xcd;
+        return SpPlace{unit < units ? unit : -1, at % row_tiles};
+    }
+    if (xcd * run + at >= units * row_tiles) return SpPlace{-1, 0};
     // the q-th unit of the order: those of residues below units % 8 are one more
-    const int q = at / row_tiles, few = units / SP_XCDS, more = units % SP_XCDS, q0 = more * (few + 1);
+    const int q = (xcd * run + at) / row_tiles, few = units / SP_XCDS, more = units % SP_XCDS, q0 = more * (few + 1);
     const int unit = q < q0 ? q % (few + 1) * SP_XCDS + q / (few + 1)
                             : (q - q0) % few * SP_XCDS + more + (q - q0) / few;
-    return SpPlace{unit, at % row_tiles};
+    return SpPlace{unit, (xcd * run + at) % row_tiles};
 }
 
 // ---- microscaled dense products past 64 rows (qmv.hip) -------------------------

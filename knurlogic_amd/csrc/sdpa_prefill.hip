@@ -32,8 +32,8 @@
 // cores busy 25%); 120 queries over 882 keys 118 -> 26 us (one launch's host
 // work instead of three).  D = 256 holds one workgroup per CU: 512 queries x 16
 // heads over 2 KV heads, 4096 keys 229 -> 129, 300 over 2000 117 -> 62.
-// Chunks of 2048 queries over 4000 keys (few units, cut over all XCDs by
-// sp_place; a unit per XCD in brackets): 32 heads over 4, D = 128 1006 -> 229 (435),
+// Chunks of 2048 queries over 4000 keys (few units, cut over all XCDs,
+// dispatch.hpp; a unit per XCD in brackets): 32 heads over 4, D = 128 1006 -> 229 (435),
 // 16 over 2, D = 256 765 -> 419 (1526).
 #include "dispatch.hpp"
 #include "qgemv_dl.hpp"
@@ -559,7 +559,7 @@ SpPlan sp_plan(int64_t BHk, int64_t rows, int64_t N, int64_t D) {
 
 template <int BITS, int D>
 int sp_go(const SpArgs& a, hipStream_t st) {
-    const int64_t wgs = (int64_t)a.BHk * a.splits * a.row_tiles + SP_XCDS;
+    const int64_t wgs = ((int64_t)a.BHk * a.splits + SP_XCDS) * a.row_tiles;
     if (wgs >= (1LL << 31)) {
         set_error("sdpa_prefill: grid of %lld workgroups", (long long)wgs);
         return EINVAL_ARG;

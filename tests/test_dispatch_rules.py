@@ -39,8 +39,8 @@ def rules(tmp_path_factory):
 
 
 @pytest.mark.parametrize("units,tiles", [(1, 1), (1, 128), (2, 128), (4, 128), (6, 3), (8, 16), (9, 5), (16, 32), (51, 1),
-                                         (3, 7)])
-def test_prompt_attention_grid_covers_every_tile_once_and_all_xcds_alike(rules, units, tiles):
+                                         (3, 7), (44, 6), (20, 16), (12, 19), (6, 128), (13, 40), (100, 3)])
+def test_prompt_attention_grid_covers_every_tile_once_and_fills_the_xcds(rules, units, tiles):
     n = 8 * rules.run(units, tiles)
     seen, load, t = set(), [0] * 8, ctypes.c_int()
     for i in range(n + 16):
@@ -51,11 +51,13 @@ def test_prompt_attention_grid_covers_every_tile_once_and_all_xcds_alike(rules, 
         seen.add((u, t.value))
         load[i % 8] += 1
     assert len(seen) == units * tiles
-    assert max(load) == -(-units * tiles // 8)          # no XCD holds more than an eighth (rounded up)
-    if units % 8 == 0:                                  # whole units per XCD
+    per_cu = lambda wgs: -(-wgs // 32)
+    even = -(-units * tiles // 8)
+    assert per_cu(max(load)) == per_cu(even)            # no CU has more to do than an even share gives
+    if per_cu(-(-units // 8) * tiles) == per_cu(even):  # whole units then
         for i in range(n):
             u = rules.place(i, units, tiles, ctypes.byref(t))
-            assert u % 8 == i % 8
+            assert u < 0 or u % 8 == i % 8
 
 
 #: measured (us): the batched kernel, the GEMM -- mxfp4, M x [N, K]
