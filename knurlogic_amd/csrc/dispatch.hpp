@@ -57,11 +57,13 @@ constexpr SpPlace sp_place(int id, int units, int row_tiles) {
 // mxfp4, batched against GEMM: 65 rows x [64, 14336] 16.1 and 20.2 us, 128 x
 // [256, 4096] 12.9 and 16.3, 65 x [1000, 4096] 14.4 and 16.3, 1000 x [64, 14336] 19.9
 // and 22.0; but 1000 x [256, 2048] 16.5 and 15.6, 65 x [1000, 14336] 27.0 and 24.3,
-// 300 x [1000, 2048] 20.3 and 17.7.  (K is not split below 1024; there the GEMM
-// is one launch for two: 65 x [64, 512] 13.0 and 11.0.)
+// 300 x [1000, 2048] 20.3 and 17.7.  At K = 1024 device time differs at twice the
+// outputs too: 129 x [1000, 1024] 12.0 and 13.8, 1000 x [256, 1024] 13.1 and 14.1.  (K is
+// not split below 1024; there the GEMM is one launch for two: 65 x [64, 512] 13.0
+// and 11.0.)
 constexpr bool mx_batched_wanted(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = rule_ceil_div(M, 64) * rule_ceil_div(N, 64);
-    return K >= 1024 && tiles <= 32 && tiles * (K / 64) <= 4000;
+    return K >= 1024 && tiles <= (K < 2048 ? 64 : 32) && tiles * (K / 64) <= 4000;
 }
 
 // ---- codebook experts: grouped GEMM or 16-row expert tiles (vq.hip, vq_packed.hip)

@@ -66,7 +66,7 @@ MX = [(65, 64, 2048, 12.9, 14.0), (65, 64, 14336, 16.1, 20.2), (128, 256, 4096, 
       (300, 64, 14336, 16.8, 20.6), (1000, 64, 14336, 19.9, 22.0),
       (65, 64, 512, 13.0, 11.0), (65, 4096, 2048, 20.2, 14.8), (1000, 256, 2048, 16.5, 15.6), (65, 1000, 14336, 27.0, 24.3),
       (300, 1000, 2048, 20.3, 17.7), (129, 1000, 4096, 18.4, 17.0), (1000, 4096, 14336, 459.5, 123.4),
-      (1000, 256, 14336, 41.7, 29.0)]
+      (1000, 256, 14336, 41.7, 29.0), (129, 1000, 1024, 12.0, 13.8), (1000, 256, 1024, 13.1, 14.1)]
 
 
 @pytest.mark.parametrize("M,N,K,batched,gemm", MX)
