@@ -78,8 +78,8 @@ constexpr int vqg_tile_rows(int code_bytes, int dim) { return 32 * vqg_max_block
 // per expert.  The GEMM wants its gate/up grid to fill CUs (g: workgroups of a
 // largest tile and 256 output columns, one per CU) and rows enough per tile, the
 // fewer the more inputs share what a tile sets up; g, rows and H trade.  The
-// lines come from 2020 calls timed on both, 4 to 128 experts, 1024..3072 -> 256..1536,
-// 3 to 400 rows; none takes the kernel that was over 2% slower.  Nearest to them,
+// lines come from 2018 calls timed on both, 4 to 128 experts, 1024..3072 -> 256..1536,
+// 3 to 400 rows; none takes the kernel that was over 3% slower.  Nearest to them,
 // 16-row tiles and GEMM, us:
 //   one-byte codes: 128 experts 2048 -> 768 (g 384), 16 rows 112 and 103; 40 experts
 //     (g 120), 47 rows 88 and 78; 32 experts (g 96), 32 rows 63 and 63; 1024 -> 512: 60
@@ -95,8 +95,11 @@ constexpr int vqg_tile_rows(int code_bytes, int dim) { return 32 * vqg_max_block
 //     32 experts (g 96), 12 rows 84 and 70; 16 experts 2048 -> 512 (g 32), 24 rows 59 and 72;
 //     1280 -> 512: 32 experts (g 64), 12 rows 50 and 56, 24 rows 63 and 60; 8 experts (g 16),
 //     48 rows 45 and 58.
-//   vectors of 2: 128 experts 2816 -> 704, 17 rows 388 and 363; 24 experts 1024 -> 512 (g
-//     48), 56 rows 67 and 75; 24 experts 2048 -> 512 (g 48), 54 rows 137 and 108.
+//   vectors of 8 (8-bit, one gather each) from fewer: 32 experts 3072 -> 512 (g 64),
+//     23 rows 117 and 80; 24 experts 2048 -> 768 (g 72), 20 rows 82 and 63.
+//   vectors of 2: 128 experts 2816 -> 704, 17 rows 388 and 363; 48 experts 3072 -> 512 (g
+//     96), 22 rows 161 and 185; 24 experts 1024 -> 512 (g 48), 56 rows 67 and 75; 24
+//     experts 2048 -> 512 (g 48), 54 rows 137 and 108.
 constexpr bool vqg_wanted(int code_bytes, int dim, int64_t P, int64_t E, int64_t avg, int64_t H, int64_t I) {
     const int64_t blocks = vqg_max_blocks(code_bytes, dim), full = avg / (32 * blocks);
     const int64_t rest = rule_ceil_div(avg - full * 32 * blocks, 32);
@@ -113,8 +116,11 @@ constexpr bool vqg_wanted(int code_bytes, int dim, int64_t P, int64_t E, int64_t
     if (code_bytes == 1)
         return P >= 1024 && ((g >= 128 && avg >= (H >= 2 * I ? 16 : 24)) || (g >= 96 && avg >= (wide ? 40 : 64)) ||
                              (wide && g >= 72 && avg >= 200));
-    if (dim == 2) return P >= 1024 && avg >= 17 && (g >= 56 || (g >= 40 && (wide || avg >= 140)));
+    if (dim == 2) return P >= 1024 && avg >= (g >= 120 ? 17 : 24) && (g >= 56 || (g >= 40 && (wide || avg >= 140)));
     if (P < 384 || avg < (P >= 640 ? 5 : 12)) return false;
+    if (dim == 8 && ((g >= 80 && avg >= 12) || (g >= 64 && avg >= 20) || (wide && g >= 40 && avg >= 20) ||
+                     (wide && g >= 24 && avg >= 100)))
+        return true;
     return g >= 128 || (g >= 96 && avg >= (wide ? 12 : 16)) || (g >= 80 && avg >= 18) || (g >= 64 && avg >= 24) ||
            (g >= (wide ? 32 : 40) && avg >= 36) || (wide && g >= 27 && avg >= 140);
 }

@@ -129,6 +129,9 @@ VQ = [
     (0, 2, 80, 1360, 2048, 512, 169.3, 149.6),
     (0, 2, 128, 3072, 1280, 512, 180.9, 131.0),
     (0, 2, 48, 5136, 1024, 256, 130.3, 74.3),
+    (0, 2, 48, 1056, 3072, 512, 161.3, 185.2),
+    (0, 8, 32, 736, 3072, 512, 117.2, 80.0),
+    (0, 8, 24, 480, 2048, 768, 82.2, 62.8),
 ]
 
 
