@@ -500,7 +500,6 @@ __global__ __launch_bounds__(256) void sdpa_merge_flat(const float* __restrict__
     for (int s = 0; s < splits; s++) m = __builtin_fmaxf(m, pm[s * rows + row].x);
     f32x4 o = {0.f, 0.f, 0.f, 0.f};
     float l = 0.f;
-#pragma unroll 4
     for (int s = 0; s < splits; s++) {
         const float2 ml = pm[s * rows + row];
         const float f = __builtin_amdgcn_exp2f((ml.x - m) * SP_LOG2E);
